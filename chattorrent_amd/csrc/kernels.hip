@@ -2885,122 +2885,217 @@ void launch_gather_rows(hipStream_t st, const float* x, const float* alt, const 
 // ==================================================================== top-k ===
 // topk_stage / topkRows (web/model/kernels.js:1453-1507, :2129-2144): per row
 // the best M (value, index) pairs, larger value first, ties to the lower
-// index. Keys pack (order-preserving value bits, ~index) so a descending
-// sort of 64-bit keys is that order; 4096 keys per workgroup are bitonic
-// sorted in LDS and the best M kept, stage after stage until one workgroup's
-// output is left.
+// index. Keys pack (order-preserving value bits, ~index), so the order of the
+// 64-bit keys is that order and no two are equal; 0 is no key. A workgroup
+// takes 4096 keys, 16 a thread, and keeps their best M in order, stage after
+// stage until one workgroup's output is left, which writes the pairs.
 __device__ static inline uint64_t topk_key(float v, uint32_t i) {
     uint32_t b = f2u(v);
     b = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
     return ((uint64_t)b << 32) | (uint64_t)(0xffffffffu - i);
 }
 
-constexpr int TOPK_CH = 4096;
+constexpr int TOPK_CH = 4096, TOPK_T = 256, TOPK_PER = TOPK_CH / TOPK_T;
 
-// A head logit: the LM-head matmul's planes added in order.
-__device__ static inline float plane_sum(const float* __restrict__ p, int planes, size_t stride, size_t i) {
-    float v = p[i];
-    for (int q = 1; q < planes; q++) v = v + p[q * stride + i];
-    return v;
+// This thread's 16 keys of the row's chunk at `base`, one of each 256 entries:
+// from the head's logits, its planes added in order with a plane's 16 loads
+// in flight at once, or from a stage's keys, which come as sorted runs of M:
+// there the entry is skewed by a step of 37 a run of 256, so that a thread's
+// keys have different ranks (at M = 256 they would all have the same one, and
+// the largest of the threads would bound the M-th badly). 0 past the end.
+__device__ static inline void topk_load(const float* __restrict__ logits, int planes, size_t stride,
+                                        const uint64_t* __restrict__ keys_in, int row, int n, int base,
+                                        uint64_t (&key)[TOPK_PER]) {
+    const int t = threadIdx.x;
+    if (!logits) {
+#pragma unroll
+        for (int j = 0; j < TOPK_PER; j++) {
+            const int i = base + j * TOPK_T + ((t + 37 * j) & (TOPK_T - 1));
+            key[j] = i < n ? keys_in[(size_t)row * n + i] : 0;
+        }
+        return;
+    }
+    const float* p = logits + (size_t)row * n;
+    float v[TOPK_PER];
+#pragma unroll
+    for (int j = 0; j < TOPK_PER; j++) {
+        const int i = base + t + j * TOPK_T;
+        v[j] = i < n ? p[i] : 0.0f;
+    }
+    for (int q = 1; q < planes; q++) {
+        p += stride;
+        float w[TOPK_PER];
+#pragma unroll
+        for (int j = 0; j < TOPK_PER; j++) {
+            const int i = base + t + j * TOPK_T;
+            w[j] = i < n ? p[i] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < TOPK_PER; j++) v[j] = v[j] + w[j];
+    }
+#pragma unroll
+    for (int j = 0; j < TOPK_PER; j++) {
+        const int i = base + t + j * TOPK_T;
+        key[j] = i < n ? topk_key(v[j], (uint32_t)i) : 0;
+    }
 }
 
-__global__ __launch_bounds__(256) void k_topk_stage(const float* __restrict__ logits, int planes,
-                                                    const uint64_t* __restrict__ keys_in, int n, int M,
-                                                    uint64_t* __restrict__ out) {
-    const size_t stride = (size_t)gridDim.y * n;
-    __shared__ uint64_t s[TOPK_CH];
-    const int row = blockIdx.y;
-    const int base = blockIdx.x * TOPK_CH;
-    for (int k = threadIdx.x; k < TOPK_CH; k += 256) {
-        const int i = base + k;
-        uint64_t key = 0;
-        if (i < n)
-            key = logits ? topk_key(plane_sum(logits, planes, stride, (size_t)row * n + i), (uint32_t)i)
-                         : keys_in[(size_t)row * n + i];
-        s[k] = key;
+// Pair or key m of a row: the last stage (vals) writes the pair, the others the key.
+__device__ static inline void topk_emit(uint64_t k, int row, int groups, int M, int m, uint64_t* __restrict__ out,
+                                        float* __restrict__ vals, uint32_t* __restrict__ ids) {
+    if (!vals) {
+        out[((size_t)row * groups + blockIdx.x) * M + m] = k;
+        return;
+    }
+    uint32_t b = (uint32_t)(k >> 32);
+    b = (b & 0x80000000u) ? (b & 0x7fffffffu) : ~b;
+    vals[(size_t)row * M + m] = u2f(b);
+    ids[(size_t)row * M + m] = 0xffffffffu - (uint32_t)(k & 0xffffffffu);
+}
+
+// How many of s[0 .. n) (n a multiple of 8, 16-byte aligned) are larger than
+// each of K keys: every thread reads the same keys, a broadcast.
+template <int K>
+__device__ static inline void topk_larger(const uint64_t* s, int n, const uint64_t (&k)[K], int (&c)[K]) {
+#pragma unroll
+    for (int i = 0; i < K; i++) c[i] = 0;
+    for (int q = 0; q < n; q += 8) {
+        ulonglong2 x[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = *(const ulonglong2*)(s + q + 2 * e);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < K; i++) c[i] += (x[e].x > k[i] ? 1 : 0) + (x[e].y > k[i] ? 1 : 0);
+    }
+}
+
+// The best M of a chunk, by elimination rather than a sort of all 4096 keys:
+// the M-th largest of the threads' largest keys is a key that at least M keys
+// reach, and few others do (M = 40: about 45 keys of 4096 in random order;
+// above 64 each thread gives the largest of each of its two halves, which
+// keeps that bound tight: about 350 at M = 256). Those that reach it are
+// gathered and ordered: up to 512 by counting, for each, the larger ones
+// (no barriers), more (an unlucky order of the input) by a bitonic sort of
+// the next power of two. What bounds it is reading the planes: at 32 rows of
+// 151936 logits in 4 planes (78 MB), M = 40, the two stages took 536 us as a
+// bitonic sort of every chunk and take 31 now; at 128 rows, M = 256, one
+// plane, the three take 204 us (1 row: 68).
+__global__ __launch_bounds__(TOPK_T) void k_topk_stage(const float* __restrict__ logits, int planes,
+                                                       const uint64_t* __restrict__ keys_in, int n, int M,
+                                                       uint64_t* __restrict__ out, float* __restrict__ vals,
+                                                       uint32_t* __restrict__ ids) {
+    __shared__ __align__(16) uint64_t s[TOPK_CH];
+    __shared__ __align__(16) uint64_t mx[2 * TOPK_T];
+    __shared__ uint64_t s_thr;
+    __shared__ int s_cnt;
+    const int t = threadIdx.x, row = blockIdx.y, groups = gridDim.x;
+    uint64_t key[TOPK_PER];
+    topk_load(logits, planes, (size_t)gridDim.y * n, keys_in, row, n, blockIdx.x * TOPK_CH, key);
+    uint64_t top[2] = {0, 0};
+#pragma unroll
+    for (int j = 0; j < TOPK_PER; j++) {
+        uint64_t& m = top[j / (TOPK_PER / 2)];
+        m = key[j] > m ? key[j] : m;
+    }
+    const bool halves = M > 64;
+    if (!halves) top[0] = top[1] > top[0] ? top[1] : top[0];
+    mx[t] = top[0];
+    if (halves) mx[TOPK_T + t] = top[1];
+    if (t == 0) {
+        s_cnt = 0;
+        s_thr = 1;   // fewer than M of the largest are keys: every key stays
     }
     __syncthreads();
-    for (int size = 2; size <= TOPK_CH; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = threadIdx.x; i < TOPK_CH; i += 256) {
-                const int l = i ^ stride;
-                if (l > i) {
-                    const bool desc = (i & size) == 0;
-                    const uint64_t a = s[i], b = s[l];
-                    if (desc ? (a < b) : (a > b)) {
-                        s[i] = b;
-                        s[l] = a;
-                    }
+    const int nm = halves ? 2 * TOPK_T : TOPK_T;
+    if (halves) {
+        int c[2];
+        topk_larger(mx, nm, top, c);
+        if (top[0] && c[0] == M - 1) s_thr = top[0];
+        if (top[1] && c[1] == M - 1) s_thr = top[1];
+    } else {
+        const uint64_t k[1] = {top[0]};
+        int c[1];
+        topk_larger(mx, nm, k, c);
+        if (top[0] && c[0] == M - 1) s_thr = top[0];
+    }
+    __syncthreads();
+    const uint64_t thr = s_thr;
+#pragma unroll
+    for (int j = 0; j < TOPK_PER; j++)
+        if (key[j] >= thr) s[atomicAdd(&s_cnt, 1)] = key[j];
+    __syncthreads();
+    const int C = s_cnt;
+    if (C <= 2 * TOPK_T) {
+        const int C8 = (C + 7) & ~7;
+        if (C + t < C8) s[C + t] = 0;
+        __syncthreads();
+        auto keep = [&](uint64_t k, int r) {
+            if (k && r < M) topk_emit(k, row, groups, M, r, out, vals, ids);
+        };
+        if (C <= TOPK_T) {
+            const uint64_t k[1] = {t < C ? s[t] : 0};
+            int c[1];
+            topk_larger(s, C8, k, c);
+            keep(k[0], c[0]);
+        } else {
+            const uint64_t k[2] = {s[t], TOPK_T + t < C ? s[TOPK_T + t] : 0};
+            int c[2];
+            topk_larger(s, C8, k, c);
+            keep(k[0], c[0]);
+            keep(k[1], c[1]);
+        }
+        for (int m = C + t; m < M; m += TOPK_T) topk_emit(0, row, groups, M, m, out, vals, ids);
+        return;
+    }
+    int n2 = 4 * TOPK_T;
+    while (n2 < C) n2 <<= 1;
+    for (int i = C + t; i < n2; i += TOPK_T) s[i] = 0;
+    __syncthreads();
+    for (int size = 2; size <= n2; size <<= 1)
+        for (int st = size >> 1; st > 0; st >>= 1) {
+            for (int p = t; p < n2 / 2; p += TOPK_T) {
+                const int i = ((p & ~(st - 1)) << 1) | (p & (st - 1)), l = i | st;
+                const uint64_t a = s[i], b = s[l];
+                if (((i & size) == 0) ? (a < b) : (a > b)) {
+                    s[i] = b;
+                    s[l] = a;
                 }
             }
             __syncthreads();
         }
-    }
-    const int groups = gridDim.x;
-    for (int m = threadIdx.x; m < M; m += 256) out[(size_t)row * groups * M + (size_t)blockIdx.x * M + m] = s[m];
-}
-
-__global__ void k_topk_unpack(const uint64_t* __restrict__ keys, int rows, int M, float* __restrict__ vals,
-                              uint32_t* __restrict__ ids) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * M) return;
-    const uint64_t k = keys[i];
-    uint32_t b = (uint32_t)(k >> 32);
-    b = (b & 0x80000000u) ? (b & 0x7fffffffu) : ~b;
-    vals[i] = u2f(b);
-    ids[i] = 0xffffffffu - (uint32_t)(k & 0xffffffffu);
+    for (int m = t; m < M; m += TOPK_T) topk_emit(s[m], row, groups, M, m, out, vals, ids);
 }
 
 // M = 1 (greedy, argmax_rows semantics: web/model/kernels.js:1411-1443): the
-// largest key of 4096 entries per workgroup, then of the workgroups' keys.
-__global__ __launch_bounds__(256) void k_argmax_stage(const float* __restrict__ logits, int planes,
-                                                      const uint64_t* __restrict__ keys_in, int n,
-                                                      uint64_t* __restrict__ out) {
-    const size_t stride = (size_t)gridDim.y * n;
-    __shared__ uint64_t red[256];
-    const int row = blockIdx.y;
-    const int base = blockIdx.x * TOPK_CH;
+// largest key of each chunk, then of the chunks' keys.
+__global__ __launch_bounds__(TOPK_T) void k_argmax_stage(const float* __restrict__ logits, int planes,
+                                                         const uint64_t* __restrict__ keys_in, int n,
+                                                         uint64_t* __restrict__ out, float* __restrict__ vals,
+                                                         uint32_t* __restrict__ ids) {
+    __shared__ uint64_t red[TOPK_T / 64];
+    const int t = threadIdx.x, row = blockIdx.y;
+    uint64_t key[TOPK_PER];
+    topk_load(logits, planes, (size_t)gridDim.y * n, keys_in, row, n, blockIdx.x * TOPK_CH, key);
     uint64_t best = 0;
-    for (int k = threadIdx.x; k < TOPK_CH; k += 256) {
-        const int i = base + k;
-        if (i >= n) break;
-        const uint64_t key = logits ? topk_key(plane_sum(logits, planes, stride, (size_t)row * n + i), (uint32_t)i)
-                                    : keys_in[(size_t)row * n + i];
-        best = key > best ? key : best;
+#pragma unroll
+    for (int j = 0; j < TOPK_PER; j++) best = key[j] > best ? key[j] : best;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint64_t x = __shfl_xor((unsigned long long)best, o);
+        best = x > best ? x : best;
     }
-    red[threadIdx.x] = best;
+    if ((t & 63) == 0) red[t >> 6] = best;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] = red[threadIdx.x + s] > red[threadIdx.x] ? red[threadIdx.x + s] : red[threadIdx.x];
-        __syncthreads();
+    if (t == 0) {
+#pragma unroll
+        for (int w = 1; w < TOPK_T / 64; w++) best = red[w] > best ? red[w] : best;
+        topk_emit(best, row, gridDim.x, 1, 0, out, vals, ids);
     }
-    if (threadIdx.x == 0) out[(size_t)row * gridDim.x + blockIdx.x] = red[0];
 }
 
 void launch_topk(hipStream_t st, const float* logits, int planes, int rows, int V, int M, uint64_t* a,
                  uint64_t* b, float* vals, uint32_t* ids) {
-    if (M == 1) {
-        int n = V;
-        const float* lg = logits;
-        const uint64_t* in = nullptr;
-        uint64_t* out = a;
-        uint64_t* other = b;
-        for (;;) {
-            const int groups = (n + TOPK_CH - 1) / TOPK_CH;
-            hipLaunchKernelGGL(k_argmax_stage, dim3(groups, rows), dim3(256), 0, st, lg, planes, in, n, out);
-            CHECK_LAUNCH();
-            if (groups == 1) break;
-            lg = nullptr;
-            in = out;
-            n = groups;
-            uint64_t* t = out;
-            out = other;
-            other = t;
-        }
-        hipLaunchKernelGGL(k_topk_unpack, dim3((rows + 255) / 256), dim3(256), 0, st, out, rows, 1, vals, ids);
-        CHECK_LAUNCH();
-        return;
-    }
     int n = V;
     const float* lg = logits;
     const uint64_t* in = nullptr;
@@ -3008,18 +3103,20 @@ void launch_topk(hipStream_t st, const float* logits, int planes, int rows, int 
     uint64_t* other = b;
     for (;;) {
         const int groups = (n + TOPK_CH - 1) / TOPK_CH;
-        hipLaunchKernelGGL(k_topk_stage, dim3(groups, rows), dim3(256), 0, st, lg, planes, in, n, M, out);
+        const bool last = groups == 1;
+        if (M == 1)
+            hipLaunchKernelGGL(k_argmax_stage, dim3(groups, rows), dim3(TOPK_T), 0, st, lg, planes, in, n, out,
+                               last ? vals : nullptr, last ? ids : nullptr);
+        else
+            hipLaunchKernelGGL(k_topk_stage, dim3(groups, rows), dim3(TOPK_T), 0, st, lg, planes, in, n, M, out,
+                               last ? vals : nullptr, last ? ids : nullptr);
         CHECK_LAUNCH();
-        if (groups == 1) break;
+        if (last) break;
         lg = nullptr;
         in = out;
         n = groups * M;
-        uint64_t* t = out;
-        out = other;
-        other = t;
+        std::swap(out, other);
     }
-    hipLaunchKernelGGL(k_topk_unpack, dim3((rows * M + 255) / 256), dim3(256), 0, st, out, rows, M, vals, ids);
-    CHECK_LAUNCH();
 }
 
 // The staged keys launch_topk needs for (rows, V, M): the first half (`a`,

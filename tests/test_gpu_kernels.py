@@ -164,6 +164,40 @@ def test_topk_exact(ctx, V, M):
         assert np.array_equal(vals[r].view(np.uint32), wv.view(np.uint32))
 
 
+@pytest.mark.parametrize("V,M", [(255, 255), (256, 64), (4095, 65), (4096, 256), (4097, 2), (16384, 64),
+                                 (20001, 256)])
+@pytest.mark.parametrize("order", ["random", "rising", "falling", "equal", "strided", "lowest"])
+def test_topk_selection_edges(ctx, V, M, order):
+    """The best-M selection where its shortcuts give out: chunks that end
+    inside a thread's keys, fewer keys than candidates asked for, M on both
+    sides of the two-halves rule, and orders that leave many keys above the
+    threads' bound (every value equal, a whole thread's column on top, rows of
+    the type's lowest values and infinities). Exact."""
+    from oracle import lib as L
+    rng = np.random.default_rng(V * 7 + M)
+    x = np.sort(rng.standard_normal(V).astype(np.float32))
+    if order == "random":
+        rng.shuffle(x)
+    elif order == "falling":
+        x = x[::-1].copy()
+    elif order == "equal":
+        x[:] = -1.5
+    elif order == "strided":      # the best keys all in a few threads' columns
+        rng.shuffle(x)
+        i = np.arange(V) % 256 < 3
+        x[i] += 100.0
+    elif order == "lowest":
+        x[:] = np.float32(-np.finfo(np.float32).max)
+        x[::3] = -np.inf
+        x[V // 2] = 0.0
+    logits = np.stack([x, x[::-1]])
+    vals, ids = ctx.op_topk(logits, M)
+    for r in range(2):
+        wv, wi = L.topk(logits[r], M)
+        assert np.array_equal(ids[r], wi)
+        assert np.array_equal(vals[r].view(np.uint32), wv.view(np.uint32))
+
+
 def test_rmsnorm_vs_oracle(ctx):
     """rmsnorm (web/model/kernels.js:930-976). The GPU sums squares four
     columns a thread, across each 64-lane wave (butterfly) and then over the
