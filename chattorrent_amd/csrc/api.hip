@@ -1402,10 +1402,10 @@ static void prof_replay(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, in
 }
 
 // k_pack over the PackJobs the pass uploaded, each past advanced by `step`.
-static void pack_on_device(cc_ctx* ctx, const MetaLayout& ml, int njobs, int step, bool head) {
+static void pack_on_device(cc_ctx* ctx, const MetaLayout& ml, int njobs, int nlaunch, int step, bool head) {
     PackGeom g{ctx->geom.nKV, ctx->group, ctx->geom.ng, ctx->D, ctx->ppw, ctx->geom.page, head ? 1 : 0};
     uint8_t* dm = ctx->d_meta;
-    launch_pack(ctx->stream, (const PackJob*)(dm + ml.pack), njobs, step, g, (JobDev*)(dm + ml.jobs),
+    launch_pack(ctx->stream, (const PackJob*)(dm + ml.pack), njobs, nlaunch, step, g, (JobDev*)(dm + ml.jobs),
                 (AttnItem*)(dm + ml.items), (int32_t*)(dm + ml.row_job), (int32_t*)(dm + ml.head_rows),
                 (int32_t*)(dm + ml.cwg));
 }
@@ -1556,7 +1556,7 @@ cc_status cc_step(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_t at, in
     hipStream_t st = ctx->stream;
     HIPCHK(hipEventRecord(ctx->ev0, st));
     HIPCHK(hipMemcpyAsync(ctx->d_meta, hm, copy_bytes, hipMemcpyHostToDevice, st));
-    pack_on_device(ctx, ml, njobs, 0, head);
+    pack_on_device(ctx, ml, njobs, p.nlaunch, 0, head);
     cc_status ps = take_pages(ctx, want, (int32_t*)(ctx->d_meta + ml.plan), (int32_t*)(hm + ml.plan), status);
     if (ps != CC_OK) {
         (void)hipStreamSynchronize(st);   // the refusal is the status reported
@@ -1749,7 +1749,7 @@ cc_status cc_decode_steps(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_
                            ctx->free_stack, pass_top[k], ctx->page_table, ctx->max_pages);
         StepPlan p;
         plan_jobs(ctx, cur.data(), njobs, p, true);
-        pack_on_device(ctx, ml, njobs, k, true);
+        pack_on_device(ctx, ml, njobs, p.nlaunch, k, true);
         if (k > 0) launch_ids_col0(st, ctx->dec_ids + (k - 1) * per, S, topk, d_ids_in);
         launch_embed(st, d_ids_in, nullptr, p.T, emb, ctx->x);
         run_blocks(ctx, p, ml, 0, d.n_layer);

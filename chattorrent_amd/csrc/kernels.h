@@ -168,8 +168,9 @@ void launch_ids_col0(hipStream_t st, const uint32_t* ids, int rows, int stride, 
 // `njobs` PackJobs (each past advanced by `step`), the job table, the
 // attention work items (kv head, m-tile, chunk of ppw pages; chunk fastest),
 // row -> job, the sampled rows and the combine's (job, kv head, m-tile)
-// triples, in the order the host planner writes them.
-void launch_pack(hipStream_t st, const PackJob* in, int njobs, int step, const PackGeom& g, JobDev* jobs,
+// triples, in the order the host planner writes them. nlaunch: the item
+// list's length (StepPlan), which sizes the launch alone.
+void launch_pack(hipStream_t st, const PackJob* in, int njobs, int nlaunch, int step, const PackGeom& g, JobDev* jobs,
                  AttnItem* items, int32_t* row_job, int32_t* head_rows, int32_t* cwg);
 // The keys launch_topk stages for (rows, V, M): a_keys for its first buffer,
 // b_keys for its second.

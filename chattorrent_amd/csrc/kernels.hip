@@ -3222,9 +3222,8 @@ void launch_ids_col0(hipStream_t st, const uint32_t* ids, int rows, int stride, 
 }
 
 // ================================================================ packing ===
-// One workgroup: per-job counts in parallel, their prefix sums in job order
-// (pack_exscan), then every job's tables written by one wave, four jobs at a
-// time. A job of n rows at past p needs ceil(n*group/16)
+// Per-job counts, their prefix sums in job order, then every job's tables. A
+// job of n rows at past p needs ceil(n*group/16)
 // Q m-tiles, ceil(ceil((p+n)/64)/ppw) chunks of pages per (kv head, m-tile),
 // one combine triple per (kv head, m-tile), and nKV*mtq*ng*128 Q-operand
 // units; each work item's softmax partial takes 16*(D+4) floats, at the
@@ -3234,92 +3233,112 @@ void launch_ids_col0(hipStream_t st, const uint32_t* ids, int rows, int stride, 
 // same pages together and the pages come from HBM once; then the jobs of
 // one m-tile: first every chunk of ppw pages, then the last, shorter chunks,
 // so the blocks a launch hands out last are the short ones (k_attn).
-constexpr int PACK_THREADS = 256;
-
-static_assert(PACK_MAX_JOBS <= 4 * PACK_THREADS, "pack_exscan takes four jobs a thread");
-// Exclusive prefix sums of v[0 .. n) in place, n <= 4 * PACK_THREADS, over the
-// whole workgroup (four consecutive values a thread, a wave scan, the waves'
-// totals in order); `total` = the sum of all n. part: PACK_THREADS / 64 ints.
-__device__ static void pack_exscan(int32_t* v, int n, int32_t* part, int& total) {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    int a[4], s = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        a[i] = 4 * t + i < n ? v[4 * t + i] : 0;
-        s += a[i];
-    }
-    int x = s;   // inclusive scan of the threads' sums across the wave
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) part[w] = x;
-    __syncthreads();
-    int off = 0;
-    total = 0;
-#pragma unroll
-    for (int k = 0; k < PACK_THREADS / 64; k++) {
-        off += k < w ? part[k] : 0;
-        total += part[k];
-    }
-    int run = off + x - s;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (4 * t + i < n) v[4 * t + i] = run;
-        run += a[i];
-    }
-    __syncthreads();   // part is reused by the next scan
-}
+//
+// Every workgroup forms the counts and all their prefix sums for itself (four
+// jobs a thread, the eight sums together through one wave scan and one
+// exchange between the waves, so two barriers); the waves of all workgroups
+// then share the tables out: a job to several waves where there are more
+// waves than jobs, else several jobs to a wave. launch_pack takes one
+// workgroup per PACK_ITEMS work items (a wave then writes about one item a
+// lane). What bounds it is latency: one workgroup with a scan per sum took
+// 11.7 us for 12 chats, 15.6 for 32, 36 for 16 verify jobs at 4k-32k tokens;
+// now 7.3, 7.4 and 7.8.
+constexpr int PACK_THREADS = 256, PACK_WAVES = PACK_THREADS / 64;
+constexpr int PACK_ITEMS = 256, PACK_BLOCKS_MAX = 64;
+static_assert(PACK_MAX_JOBS <= 4 * PACK_THREADS, "four jobs a thread");
 
 __global__ __launch_bounds__(PACK_THREADS) void k_pack(const PackJob* __restrict__ in, int njobs, int step,
                                                        PackGeom g, JobDev* __restrict__ jobs,
                                                        AttnItem* __restrict__ items, int32_t* __restrict__ row_job,
                                                        int32_t* __restrict__ head_rows, int32_t* __restrict__ cwg) {
+    // per job: the sums before it (rows, items, combine triples, Q units, head
+    // rows), its place in the item list (and of its short chunks), and its counts
     __shared__ int32_t s_row0[PACK_MAX_JOBS], s_item0[PACK_MAX_JOBS], s_cwg0[PACK_MAX_JOBS],
         s_qp0[PACK_MAX_JOBS], s_head0[PACK_MAX_JOBS], s_mtq[PACK_MAX_JOBS], s_nch[PACK_MAX_JOBS],
-        s_pos0[PACK_MAX_JOBS], s_posf[PACK_MAX_JOBS], s_posb[PACK_MAX_JOBS], s_part[PACK_THREADS / 64];
-    // each job's counts, then their exclusive prefix sums in job order
-    for (int j = threadIdx.x; j < njobs; j += blockDim.x) {
-        const int n = in[j].n, tact = in[j].past + step + n;
-        const int mtq = (n * g.group + 15) / 16, pages = (tact + g.page - 1) / g.page;
-        const int nch = (pages + g.ppw - 1) / g.ppw;
-        s_mtq[j] = mtq;
-        s_nch[j] = nch;
-        s_row0[j] = n;
-        s_item0[j] = g.nKV * mtq * nch;
-        s_cwg0[j] = g.nKV * mtq;
-        s_qp0[j] = g.nKV * mtq * g.ng * 128;
-        s_head0[j] = g.head ? in[j].sampled : 0;
-        // the item list: jobs of several m-tiles first, then the one-m-tile jobs'
-        // full chunks, then their short last chunks
-        s_pos0[j] = mtq > 1 ? g.nKV * nch * 4 * ((mtq + 3) / 4) : 0;
-        s_posf[j] = mtq > 1 ? 0 : g.nKV * (pages / g.ppw);
-        s_posb[j] = mtq > 1 ? 0 : g.nKV * (pages % g.ppw != 0);
-    }
-    __syncthreads();
-    int tot_multi, tot_full, unused;
-    pack_exscan(s_row0, njobs, s_part, unused);
-    pack_exscan(s_item0, njobs, s_part, unused);
-    pack_exscan(s_cwg0, njobs, s_part, unused);
-    pack_exscan(s_qp0, njobs, s_part, unused);
-    pack_exscan(s_head0, njobs, s_part, unused);
-    pack_exscan(s_pos0, njobs, s_part, tot_multi);
-    pack_exscan(s_posf, njobs, s_part, tot_full);
-    pack_exscan(s_posb, njobs, s_part, unused);
-    for (int j = threadIdx.x; j < njobs; j += blockDim.x)
-        if (s_mtq[j] == 1) {
-            s_pos0[j] = tot_multi + s_posf[j];
-            s_posb[j] += tot_multi + tot_full;
+        s_pos0[PACK_MAX_JOBS], s_posb[PACK_MAX_JOBS], s_part[PACK_WAVES][8];
+    const int t = threadIdx.x, ln = t & 63, wv = t >> 6;
+    {
+        constexpr int NS = 8;   // rows, items, triples, Q units, head rows, list places: multi, full, short
+        int a[4][NS], mtq[4], x[NS];
+#pragma unroll
+        for (int k = 0; k < NS; k++) x[k] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int j = 4 * t + i;
+            mtq[i] = 0;
+#pragma unroll
+            for (int k = 0; k < NS; k++) a[i][k] = 0;
+            if (j < njobs) {
+                const PackJob pj = in[j];
+                const int tact = pj.past + step + pj.n, pages = (tact + g.page - 1) / g.page;
+                const int nch = (pages + g.ppw - 1) / g.ppw;
+                mtq[i] = (pj.n * g.group + 15) / 16;
+                const bool multi = mtq[i] > 1;
+                a[i][0] = pj.n;
+                a[i][1] = g.nKV * mtq[i] * nch;
+                a[i][2] = g.nKV * mtq[i];
+                a[i][3] = g.nKV * mtq[i] * g.ng * 128;
+                a[i][4] = g.head ? pj.sampled : 0;
+                a[i][5] = multi ? g.nKV * nch * 4 * ((mtq[i] + 3) / 4) : 0;
+                a[i][6] = multi ? 0 : g.nKV * (pages / g.ppw);
+                a[i][7] = multi ? 0 : g.nKV * (pages % g.ppw != 0);
+                s_mtq[j] = mtq[i];
+                s_nch[j] = nch;
+            }
+#pragma unroll
+            for (int k = 0; k < NS; k++) x[k] += a[i][k];
         }
-    __syncthreads();
+        int run[NS];   // the exclusive prefix of this thread's first job
+#pragma unroll
+        for (int k = 0; k < NS; k++) run[k] = -x[k];
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+            for (int k = 0; k < NS; k++) {
+                const int y = __shfl_up(x[k], o);
+                if (ln >= o) x[k] += y;
+            }
+        if (ln == 63)
+#pragma unroll
+            for (int k = 0; k < NS; k++) s_part[wv][k] = x[k];
+        __syncthreads();
+        int tot_multi = 0, tot_full = 0;
+#pragma unroll
+        for (int w = 0; w < PACK_WAVES; w++) {
+            tot_multi += s_part[w][5];
+            tot_full += s_part[w][6];
+#pragma unroll
+            for (int k = 0; k < NS; k++) run[k] += w < wv ? s_part[w][k] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < NS; k++) run[k] += x[k];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int j = 4 * t + i;
+            if (j < njobs) {
+                s_row0[j] = run[0];
+                s_item0[j] = run[1];
+                s_cwg0[j] = run[2];
+                s_qp0[j] = run[3];
+                s_head0[j] = run[4];
+                s_pos0[j] = mtq[i] > 1 ? run[5] : tot_multi + run[6];
+                s_posb[j] = tot_multi + tot_full + run[7];
+            }
+#pragma unroll
+            for (int k = 0; k < NS; k++) run[k] += a[i][k];
+        }
+        __syncthreads();
+    }
     const int part = 16 * (g.D + 4);
-    // one wave a job: the four waves write four jobs' tables at a time
-    const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
-    for (int j = wv; j < njobs; j += PACK_THREADS / 64) {
+    // waves in groups of wpj (1 when there are at least as many jobs as waves); a group takes every ngr-th job
+    const int nw = gridDim.x * PACK_WAVES, wpj = nw > njobs ? nw / njobs : 1, ngr = nw / wpj;
+    const int gw = blockIdx.x * PACK_WAVES + wv, sub = gw % wpj;
+    if (gw >= ngr * wpj) return;
+    const int x0 = sub * 64 + ln, dx = wpj * 64;
+    for (int j = gw / wpj; j < njobs; j += ngr) {
         const PackJob pj = in[j];
         const int past = pj.past + step, mtq = s_mtq[j], nch = s_nch[j];
-        if (ln == 0) {
+        if (x0 == 0) {
             JobDev jd;
             jd.slot = pj.slot;
             jd.past = past;
@@ -3335,7 +3354,7 @@ __global__ __launch_bounds__(PACK_THREADS) void k_pack(const PackJob* __restrict
         }
         if (mtq == 1) {
             const int nfull = ((past + pj.n + g.page - 1) / g.page) / g.ppw;
-            for (int x = ln; x < g.nKV * nch; x += 64) {
+            for (int x = x0; x < g.nKV * nch; x += dx) {
                 const int c = x % nch, h = x / nch;
                 const int idx = s_item0[j] + x;   // (kv head, m-tile 0, chunk)
                 items[c < nfull ? s_pos0[j] + h * nfull + c : s_posb[j] + h] =
@@ -3344,7 +3363,7 @@ __global__ __launch_bounds__(PACK_THREADS) void k_pack(const PackJob* __restrict
         } else {
             // (kv head, chunk, block of 4 m-tiles, m-tile): a block is one workgroup
             const int nb = (mtq + 3) / 4, nit = g.nKV * nch * nb * 4;
-            for (int x = ln; x < nit; x += 64) {
+            for (int x = x0; x < nit; x += dx) {
                 const int q = x % 4, b = (x / 4) % nb, c = (x / (4 * nb)) % nch, h = x / (4 * nb * nch);
                 const int mt = 4 * b + q;
                 if (mt >= mtq) {
@@ -3357,23 +3376,24 @@ __global__ __launch_bounds__(PACK_THREADS) void k_pack(const PackJob* __restrict
                     AttnItem{pj.slot, past, pj.n, mt, s_qp0[j] + (hm * g.ng) * 128, idx * part, h, c * g.ppw};
             }
         }
-        for (int x = ln; x < g.nKV * mtq; x += 64) {
+        for (int x = x0; x < g.nKV * mtq; x += dx) {
             const int at = 3 * (s_cwg0[j] + x);
             cwg[at] = j;
             cwg[at + 1] = x / mtq;
             cwg[at + 2] = x % mtq;
         }
-        for (int i = ln; i < pj.n; i += 64) row_job[s_row0[j] + i] = j;
+        for (int i = x0; i < pj.n; i += dx) row_job[s_row0[j] + i] = j;
         if (g.head)
-            for (int i = ln; i < pj.sampled; i += 64)
+            for (int i = x0; i < pj.sampled; i += dx)
                 head_rows[s_head0[j] + i] = s_row0[j] + pj.n - pj.sampled + i;
     }
 }
 
-void launch_pack(hipStream_t st, const PackJob* in, int njobs, int step, const PackGeom& g, JobDev* jobs,
+void launch_pack(hipStream_t st, const PackJob* in, int njobs, int nlaunch, int step, const PackGeom& g, JobDev* jobs,
                  AttnItem* items, int32_t* row_job, int32_t* head_rows, int32_t* cwg) {
     if (njobs <= 0 || njobs > PACK_MAX_JOBS) return;
-    hipLaunchKernelGGL(k_pack, dim3(1), dim3(PACK_THREADS), 0, st, in, njobs, step, g, jobs, items, row_job,
+    const int blocks = std::max(1, std::min(PACK_BLOCKS_MAX, (nlaunch + PACK_ITEMS - 1) / PACK_ITEMS));
+    hipLaunchKernelGGL(k_pack, dim3(blocks), dim3(PACK_THREADS), 0, st, in, njobs, step, g, jobs, items, row_job,
                        head_rows, cwg);
     CHECK_LAUNCH();
 }

@@ -204,6 +204,38 @@ def test_batched_equals_alone_bitwise(smol):
         at += n
 
 
+@pytest.mark.parametrize("njobs,longest,nverify", [(1, 12000, 1), (3, 9000, 2), (70, 3000, 5), (600, 400, 40)])
+def test_packed_by_many_workgroups_equals_alone(gpu, njobs, longest, nverify):
+    """The packer's tables do not depend on how many workgroups and waves share
+    the writing: several waves a job, several jobs a wave, jobs of one and of
+    several m-tiles mixed. Every sampled job of the pass gets the bits it gets
+    alone (where one or few workgroups pack it)."""
+    from chattorrent_amd.ccdecode import Context
+    rng = np.random.default_rng(njobs)
+    d = configs.with_layers(configs.SMOLLM2, 1)
+    past = np.round(np.exp(rng.uniform(0, np.log(longest), njobs))).astype(int)
+    past[0] = longest
+    n_max = 64 * (longest // 64 + 2)
+    c = Context(d, n_max=n_max, t_max=njobs + 8 * nverify + 8, slots=int((past // 64 + 2).sum() * 64 // n_max + 1),
+                sessions=njobs)
+    try:
+        c.fill_random(SEED)
+        for s, T in enumerate(past):
+            c.fill_random_kv(s, int(T), SEED, s + 1)
+        verify = set(rng.choice(njobs, nverify, replace=False).tolist()) | {0}
+        jobs = [dict(slot=s, past=int(T), n=8 if s in verify and nverify > 1 or njobs == 1 else 1, sampled=1)
+                for s, T in enumerate(past)]
+        for j in jobs:
+            j["ids"] = _ids(j["n"], d["vocab"], 100 + j["slot"])
+        vals, ids = c.step(jobs, topk=4)
+        for s in sorted(verify | set(rng.choice(njobs, min(njobs, 12), replace=False).tolist()) | {njobs - 1}):
+            v1, i1 = c.step([jobs[s]], topk=4)
+            assert np.array_equal(i1[0], ids[s]), s
+            assert np.array_equal(v1[0].view(np.uint32), vals[s].view(np.uint32)), s
+    finally:
+        c.close()
+
+
 def test_verify_rows_equal_one_row_jobs(smol):
     """docs/model.md 'Matching plain decoding row by row': row i of an 8-row
     verify gives the bits of a one-row job at past + i."""
