@@ -1293,7 +1293,7 @@ static void run_blocks(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, int
             else
                 launch_lin_conv(st, ctx->part, gemm_planes(L.lin, T, ctx->ncu), T, pm.njobs, pm.jobs, rs, L.conv, lg, L.state, ctx->lraw,
                                 ctx->lrep);
-            launch_gdn(st, ctx->lraw, ctx->lrep, pm.njobs, pm.jobs, L.gp, lg, L.state, ctx->lcore);
+            launch_gdn(st, ctx->lraw, ctx->lrep, pm.njobs, pm.jobs, L.gp, lg, L.state, ctx->lcore, longest);
             launch_lin_norm(st, ctx->lcore, ctx->lraw, L.gnorm, d.rms_eps, T, lg, L.out.KU, ctx->xp_v);
             launch_gemm(st, L.out, ctx->xp_v, ctx->mt_alloc, ctx->part, T, ctx->ncu);
             launch_resid_w(st, ctx->x, ctx->part, gemm_planes(L.out, T, ctx->ncu), T, Mpad, H, 0, L.ln2, KUH, ctx->xp_h, ctx->ssp);

@@ -1837,106 +1837,170 @@ void launch_lin_conv_rows(hipStream_t st, const float* part, int splits, int M, 
 }
 
 // gated_delta_net_step (kernels.js:1672-1805) for every row of a job, on its
-// session's S [nV][Dk][Dv]: one workgroup per (value-column tile, value head,
-// job), GDN_KS k-groups x GDN_TV columns; each thread holds DK/GDN_KS rows of
-// its column for the whole job. Per token, in the reference's arithmetic:
+// session's S [nV][Dk][Dv]. Per token, with the l2norm of the head's q and k
+// (l2norm_heads, kernels.js:1622-1670; source head h / group, the value-head
+// repeat) folded in as k^ = k/sqrt(sum k^2 + 1e-6) and q^ likewise, times
+// 1/sqrt(Dk):
 //   g = exp(-exp(A_log) * softplus(a + dt_bias)), beta = sigmoid(b);
-//   s *= g; kv = s.k, qo = s.q over k; kq = k.q;
-//   delta = (v - kv) * beta; s += k * delta; out = (qo + delta*kq) / sqrt(Dk).
-// l2norm_heads (kernels.js:1622-1670) of the head's q and k (source head
-// h / group, the value-head repeat) is folded in: the raw dot products and
-// the sums of squares share the token's one reduction through LDS (double
-// buffered on token parity, one barrier a token), and the factors
-// 1/sqrt(sum x^2 + 1e-6) are applied after it; the state update uses the
-// normalised k. A job at position 0 starts from a zero state. A rollback
-// job starts from the snapshot and first re-runs the kept rows (from `lrep`,
-// no output); a verify writes the state it starts from to the snapshot.
-constexpr int GDN_KS = 8, GDN_TV = 32;
+//   delta = (v - g*(s.k^)) * beta; out = g*(s.q^) + delta*(k^.q^);
+//   s = g*s + k^*delta.
+// A job at position 0 starts from a zero state. A rollback job starts from
+// the snapshot and first re-runs the kept rows (from `lrep`, no output); a
+// verify writes the state it starts from to the snapshot.
+//
+// A workgroup serves (32 value columns, value head, job), eight threads a
+// column with DK/8 rows of it each, in registers for the whole job. Two
+// kernels, the same operations on the same operands in the same order, so a
+// row's bits depend on neither its job's length nor its batch-mates:
+//   k_gdn_few  a pass whose jobs have few rows (GDN_FEW): bound by the state's
+//              read and write, so few registers (many workgroups to hide the
+//              reads), whole 128-byte rows of state a load, the columns' sums
+//              through LDS with a barrier a token;
+//   k_gdn      longer jobs: bound by the chain from token to token, so a
+//              column's eight threads are neighbouring lanes and its sums DPP
+//              adds with no barrier, and what a token needs that does not
+//              depend on the state (k^, q^, k^.q^, g, beta, the columns' v) is
+//              formed GDN_CH tokens at a time, a token a wave, and read
+//              from LDS a token ahead; the next tokens' inputs load under the
+//              walk.
+// A single kernel that formed the dot products of q and k beside the state's
+// and read each token's inputs as it came to them took 1.49 us a row of a
+// long job: 512 rows 759 us a block (48 heads of 128 x 128), now 203. 16
+// sessions at 1, 2, 3, 4 and 8 rows (of 3.3 MB read and twice written with
+// a verify's snapshot) took 31.6, 35.9, 41.6, 46.2 and 69.4 us; k_gdn_few
+// takes 32.7, 36.1, 41.0 and 46.0, k_gdn 50.9 at 3 and 4 rows and 55.2 at 8:
+// the line between them.
+constexpr int GDN_TV = 32, GDN_T = 256, GDN_CH = 16, GDN_KG = 8, GDN_FEW = 4;
+static_assert(LIN_SPEC_ROWS < GDN_CH, "a rollback's kept rows and the row after them fall in one chunk");
+// Sum over the eight lanes 8i .. 8i+7, in all of them:
+// ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7)).
+__device__ static inline float sum8(float x) {
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xf, 0xf, true));   // lane ^ 1
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xf, 0xf, true));   // lane ^ 2
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xf, 0xf, true));  // 7 - lane of the eight
+    return x;
+}
+// A token's inputs across a wave: q and k of the head, lane l holding
+// channels l and l + 64, and their sums of squares and product.
 template <int DK>
-__global__ __launch_bounds__(GDN_KS * GDN_TV) void k_gdn(const float* __restrict__ lraw, const float* __restrict__ lrep,
-                                                         const JobDev* __restrict__ jobs,
-                                                         const float* __restrict__ gp, LinGeom lg,
-                                                         float* __restrict__ state, float* __restrict__ core) {
-    constexpr int ROWS = DK / GDN_KS;
-    __shared__ float pkv[2][GDN_KS][GDN_TV];
-    __shared__ float pqo[2][GDN_KS][GDN_TV];
-    __shared__ float psc[2][GDN_KS][3];   // k.q, q.q, k.k per k-group
-    const int h = blockIdx.y;
-    const int j = blockIdx.z;
+struct GdnRow {
+    static constexpr int PER = (DK + 63) / 64;
+    float q[PER], k[PER];
+};
+template <int DK>
+__device__ static inline void gdn_load(GdnRow<DK>& x, const float* row, int keyDim, int kh, int lane) {
+#pragma unroll
+    for (int e = 0; e < GdnRow<DK>::PER; e++) {
+        const int d = lane + 64 * e;
+        x.q[e] = d < DK ? row[kh * DK + d] : 0.0f;
+        x.k[e] = d < DK ? row[keyDim + kh * DK + d] : 0.0f;
+    }
+}
+// q.q, k.k and k.q of T tokens, their sums across the wave side by side.
+template <int DK, int T>
+__device__ static inline void gdn_norms(const GdnRow<DK> (&x)[T], float (&n3)[T][3]) {
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+        n3[t][0] = n3[t][1] = n3[t][2] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < GdnRow<DK>::PER; e++) {
+            n3[t][0] = __builtin_fmaf(x[t].q[e], x[t].q[e], n3[t][0]);
+            n3[t][1] = __builtin_fmaf(x[t].k[e], x[t].k[e], n3[t][1]);
+            n3[t][2] = __builtin_fmaf(x[t].k[e], x[t].q[e], n3[t][2]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) n3[t][i] = sum8(n3[t][i]);
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+        for (int t = 0; t < T; t++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) n3[t][i] += __shfl_xor(n3[t][i], o);
+}
+// The factors of q and k, from their sums: q's carries 1/sqrt(Dk).
+struct GdnScale {
+    float rq, rk, kq, g, beta;
+};
+__device__ static inline GdnScale gdn_scale(const float (&n3)[3], float q_scale, float A, float dtb, float a, float b) {
+    GdnScale r;
+    r.rq = q_scale / sqrtf(n3[0] + 1e-6f);
+    r.rk = 1.0f / sqrtf(n3[1] + 1e-6f);
+    r.kq = n3[2] * r.rq * r.rk;
+    const float x = a + dtb;
+    const float sp = x > 20.0f ? x + logf(1.0f + expf(-x)) : logf(1.0f + expf(x));
+    r.g = expf(-A * sp);
+    r.beta = 1.0f / (1.0f + expf(-b));
+    return r;
+}
+
+template <int DK>
+__global__ __launch_bounds__(GDN_T) void k_gdn_few(const float* __restrict__ lraw, const float* __restrict__ lrep,
+                                                   const JobDev* __restrict__ jobs, const float* __restrict__ gp,
+                                                   LinGeom lg, float* __restrict__ state, float* __restrict__ core) {
+    constexpr int ROWS = DK / GDN_KG;
+    __shared__ float pkv[2][GDN_KG][GDN_TV], pqo[2][GDN_KG][GDN_TV];
+    const int h = blockIdx.y, j = blockIdx.z;
     const JobDev jb = jobs[j];
-    const int col = threadIdx.x % GDN_TV, kg = threadIdx.x / GDN_TV;
+    const int lane = threadIdx.x & 63, col = threadIdx.x % GDN_TV, kg = threadIdx.x / GDN_TV;
     const int vv = blockIdx.x * GDN_TV + col;
     const bool live = vv < lg.Dv;
     const int vvc = live ? vv : lg.Dv - 1;   // out-of-range columns read a real one and discard it
-    const int k0 = kg * ROWS;
-    const int kh = h / lg.group;
-    float* base = state + (size_t)jb.slot * lg.sstride + (size_t)h * DK * lg.Dv;
-    float* S = base;                // current
-    float* Ssnap = base + lg.blk;   // snapshot
+    const int k0 = kg * ROWS, kh = h / lg.group;
+    float* S = state + (size_t)jb.slot * lg.sstride + (size_t)h * DK * lg.Dv;   // current
+    float* Ssnap = S + lg.blk;                                                   // snapshot
     const float* src = jb.keep >= 0 ? Ssnap : S;
     float s[ROWS];
 #pragma unroll
     for (int i = 0; i < ROWS; i++) s[i] = (jb.past > 0 && live) ? src[(size_t)(k0 + i) * lg.Dv + vv] : 0.0f;
     const float A = expf(gp[h]), dtb = gp[lg.nV + h];
     const float q_scale = 1.0f / sqrtf((float)DK);
-    int t = 0;   // tokens so far: the LDS buffers alternate on its parity
-    // One token: q, k, v at their channel offsets in `row`, b and a at
-    // boff + h and boff + nV + h. Every thread reaches its one barrier.
-    auto token = [&](const float* row, int boff, float* out) {
-        const float* qr = row + kh * DK;
-        const float* kr = row + lg.keyDim + kh * DK;
-        const float a = row[boff + lg.nV + h] + dtb;
-        const float sp = a > 20.0f ? a + logf(1.0f + expf(-a)) : logf(1.0f + expf(a));
-        const float g = expf(-A * sp);
-        const float beta = 1.0f / (1.0f + expf(-row[boff + h]));
-        const int buf = t & 1;
-        float kv = 0.0f, qo = 0.0f, kq = 0.0f, qq = 0.0f, kk = 0.0f;
-        float kx[ROWS];
+    const int keep = jb.keep > 0 ? jb.keep : 0, total = keep + jb.n;   // the kept rows first, then the job's
+    const float* lr = lrep + (size_t)j * LIN_SPEC_ROWS * lg.lrep_w;
+    for (int t = 0; t < total; t++) {
+        const int i = t - keep;   // the job's row, < 0: a kept one
+        const float* row = i < 0 ? lr + (size_t)t * lg.lrep_w : lraw + (size_t)(jb.row0 + i) * lg.W;
+        const int boff = i < 0 ? lg.convDim : lg.convDim + lg.valueDim;
+        GdnRow<DK> x[1];
+        gdn_load<DK>(x[0], row, lg.keyDim, kh, lane);
+        float kx[ROWS], qx[ROWS];
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
-            const float ki = kr[k0 + r], qi = qr[k0 + r];
-            kx[r] = ki;
-            s[r] = s[r] * g;
-            kv = kv + s[r] * ki;
-            qo = qo + s[r] * qi;
-            kq = kq + ki * qi;
-            qq = qq + qi * qi;
-            kk = kk + ki * ki;
+            qx[r] = row[kh * DK + k0 + r];
+            kx[r] = row[lg.keyDim + kh * DK + k0 + r];
         }
-        pkv[buf][kg][col] = kv;
-        pqo[buf][kg][col] = qo;
-        if (col == 0) {
-            psc[buf][kg][0] = kq;
-            psc[buf][kg][1] = qq;
-            psc[buf][kg][2] = kk;
+        const float v = row[2 * lg.keyDim + h * lg.Dv + vvc], b = row[boff + h], a = row[boff + lg.nV + h];
+        if (i == 0 && jb.snap && live) {
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) Ssnap[(size_t)(k0 + r) * lg.Dv + vv] = s[r];
         }
+        float n3[1][3];
+        gdn_norms<DK, 1>(x, n3);
+        const GdnScale sc = gdn_scale(n3[0], q_scale, A, dtb, a, b);
+        float kv[2] = {0.0f, 0.0f}, qo[2] = {0.0f, 0.0f};   // even and odd rows
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            kx[r] = kx[r] * sc.rk;
+            kv[r & 1] = __builtin_fmaf(s[r], kx[r], kv[r & 1]);
+            qo[r & 1] = __builtin_fmaf(s[r], qx[r] * sc.rq, qo[r & 1]);
+        }
+        const int buf = t & 1;
+        pkv[buf][kg][col] = kv[0] + kv[1];
+        pqo[buf][kg][col] = qo[0] + qo[1];
         __syncthreads();
-        float kvT = 0.0f, qoT = 0.0f, kqT = 0.0f, qqT = 0.0f, kkT = 0.0f;
+        auto tree = [&](const float (&p)[GDN_KG][GDN_TV]) {   // sum8's order
+            return ((p[0][col] + p[1][col]) + (p[2][col] + p[3][col])) +
+                   ((p[4][col] + p[5][col]) + (p[6][col] + p[7][col]));
+        };
+        const float kvT = tree(pkv[buf]);
+        const float delta = (v - sc.g * kvT) * sc.beta;
 #pragma unroll
-        for (int q = 0; q < GDN_KS; q++) {
-            kvT = kvT + pkv[buf][q][col];
-            qoT = qoT + pqo[buf][q][col];
-            kqT = kqT + psc[buf][q][0];
-            qqT = qqT + psc[buf][q][1];
-            kkT = kkT + psc[buf][q][2];
-        }
-        const float rq = 1.0f / sqrtf(qqT + 1e-6f), rk = 1.0f / sqrtf(kkT + 1e-6f);
-        const float delta = (row[2 * lg.keyDim + h * lg.Dv + vvc] - kvT * rk) * beta;
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) s[r] = s[r] + (kx[r] * rk) * delta;
-        if (out && kg == 0 && live) *out = (qoT * rq + delta * (kqT * rq * rk)) * q_scale;
-        t++;
-    };
-    // a rollback re-runs the kept rows of the session's last verify
-    const float* lr = lrep + (size_t)j * LIN_SPEC_ROWS * lg.lrep_w;
-    for (int i = 0; i < jb.keep; i++) token(lr + (size_t)i * lg.lrep_w, lg.convDim, nullptr);
-    if (jb.snap && live) {
-#pragma unroll
-        for (int i = 0; i < ROWS; i++) Ssnap[(size_t)(k0 + i) * lg.Dv + vv] = s[i];
-    }
-    for (int i = 0; i < jb.n; i++) {
-        const int m = jb.row0 + i;
-        token(lraw + (size_t)m * lg.W, lg.convDim + lg.valueDim, core + (size_t)m * lg.valueDim + h * lg.Dv + vv);
+        for (int r = 0; r < ROWS; r++) s[r] = __builtin_fmaf(sc.g, s[r], kx[r] * delta);
+        if (i >= 0 && kg == 0 && live)
+            core[(size_t)(jb.row0 + i) * lg.valueDim + h * lg.Dv + vv] =
+                __builtin_fmaf(sc.g, tree(pqo[buf]), delta * sc.kq);
     }
     if (live) {
 #pragma unroll
@@ -1944,15 +2008,172 @@ __global__ __launch_bounds__(GDN_KS * GDN_TV) void k_gdn(const float* __restrict
     }
 }
 
+template <int DK>
+__global__ __launch_bounds__(GDN_T, 3) void k_gdn(const float* __restrict__ lraw, const float* __restrict__ lrep,
+                                                  const JobDev* __restrict__ jobs, const float* __restrict__ gp,
+                                                  LinGeom lg, float* __restrict__ state, float* __restrict__ core) {
+    // a lane group's ROWS values start 4 floats further than the last group's
+    // end at DK = 128, so the eight groups' 16-byte reads fall in different banks
+    constexpr int ROWS = DK / GDN_KG, LROW = ROWS == 16 ? 20 : ROWS, LK = LROW * GDN_KG;
+    constexpr int TPW = GDN_CH / (GDN_T / 64);   // tokens a wave
+    __shared__ __align__(16) float s_k[GDN_CH][LK], s_q[GDN_CH][LK], s_v[GDN_CH][GDN_TV];
+    __shared__ __align__(16) float s_sc[GDN_CH][4];   // g, beta, k^.q^
+    const int h = blockIdx.y, j = blockIdx.z;
+    const JobDev jb = jobs[j];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = lane & 7, cw = wave * 8 + (lane >> 3);
+    const int vv = blockIdx.x * GDN_TV + cw;
+    const bool live = vv < lg.Dv;
+    const int k0 = kg * ROWS, kh = h / lg.group;
+    float* S = state + (size_t)jb.slot * lg.sstride + (size_t)h * DK * lg.Dv;   // current
+    float* Ssnap = S + lg.blk;                                                   // snapshot
+    // the lane's elements through one offset register (a lane past Dv reads and
+    // writes past the resource's end: zero, dropped)
+    const int sb = DK * lg.Dv * 4, so = live ? (k0 * lg.Dv + vv) * 4 : sb;
+    float s[ROWS];
+    {
+        const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)(jb.keep >= 0 ? Ssnap : S), 0, jb.past > 0 ? sb : 0,
+                                                         0x00020000);
+#pragma unroll
+        for (int i = 0; i < ROWS; i++)
+            s[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, so, i * lg.Dv * 4, 0));
+    }
+    auto put_state = [&](float* to) {
+        const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)to, 0, sb, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < ROWS; i++)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s[i]), r, so, i * lg.Dv * 4, 0);
+    };
+    const float A = expf(gp[h]), dtb = gp[lg.nV + h];
+    const float q_scale = 1.0f / sqrtf((float)DK);
+    const int keep = jb.keep > 0 ? jb.keep : 0, total = keep + jb.n;   // the kept rows first, then the job's
+    const float* lr = lrep + (size_t)j * LIN_SPEC_ROWS * lg.lrep_w;
+    // this wave's tokens of the chunk at t0: wave, wave + 4, ...
+    GdnRow<DK> x[TPW];
+    float vr[TPW], ar[TPW], br[TPW];
+    auto load = [&](int t0) {
+#pragma unroll
+        for (int u = 0; u < TPW; u++) {
+            const int i = min(t0 + wave + u * (GDN_T / 64), total - 1);   // past the end: loaded and not used
+            const float* row = i < keep ? lr + (size_t)i * lg.lrep_w : lraw + (size_t)(jb.row0 + i - keep) * lg.W;
+            const int boff = i < keep ? lg.convDim : lg.convDim + lg.valueDim;
+            gdn_load<DK>(x[u], row, lg.keyDim, kh, lane);
+            const int c = blockIdx.x * GDN_TV + (lane & (GDN_TV - 1));
+            vr[u] = row[2 * lg.keyDim + h * lg.Dv + (c < lg.Dv ? c : lg.Dv - 1)];
+            br[u] = row[boff + h];
+            ar[u] = row[boff + lg.nV + h];
+        }
+    };
+    auto prepare = [&](int t0) {
+        float n3[TPW][3];
+        gdn_norms<DK, TPW>(x, n3);
+#pragma unroll
+        for (int u = 0; u < TPW; u++) {
+            const int c = wave + u * (GDN_T / 64);
+            if (t0 + c >= total) continue;
+            const GdnScale sc = gdn_scale(n3[u], q_scale, A, dtb, ar[u], br[u]);
+#pragma unroll
+            for (int e = 0; e < GdnRow<DK>::PER; e++) {
+                const int d = lane + 64 * e;
+                if (d < DK) {
+                    const int at = (d / ROWS) * LROW + d % ROWS;
+                    s_q[c][at] = x[u].q[e] * sc.rq;
+                    s_k[c][at] = x[u].k[e] * sc.rk;
+                }
+            }
+            if (lane < GDN_TV) s_v[c][lane] = vr[u];
+            if (lane == 0) *(float4*)s_sc[c] = make_float4(sc.g, sc.beta, sc.kq, 0.0f);
+        }
+    };
+    struct Tok {
+        float k[ROWS], q[ROWS], v;
+        float4 sc;
+    };
+    auto fetch = [&](Tok& y, int c) {
+        if constexpr (ROWS >= 4) {
+#pragma unroll
+            for (int r = 0; r < ROWS; r += 4) {
+                const float4 ka = *(const float4*)&s_k[c][kg * LROW + r], qa = *(const float4*)&s_q[c][kg * LROW + r];
+                y.k[r] = ka.x; y.k[r + 1] = ka.y; y.k[r + 2] = ka.z; y.k[r + 3] = ka.w;
+                y.q[r] = qa.x; y.q[r + 1] = qa.y; y.q[r + 2] = qa.z; y.q[r + 3] = qa.w;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                y.k[r] = s_k[c][kg * LROW + r];
+                y.q[r] = s_q[c][kg * LROW + r];
+            }
+        }
+        y.sc = *(const float4*)s_sc[c];
+        y.v = s_v[c][cw];
+    };
+    auto advance = [&](const Tok& y, float* o) {
+        float kv[2] = {0.0f, 0.0f}, qo[2] = {0.0f, 0.0f};   // even and odd rows
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            kv[r & 1] = __builtin_fmaf(s[r], y.k[r], kv[r & 1]);
+            qo[r & 1] = __builtin_fmaf(s[r], y.q[r], qo[r & 1]);
+        }
+        const float kvT = sum8(kv[0] + kv[1]), qoT = sum8(qo[0] + qo[1]);
+        const float delta = (y.v - y.sc.x * kvT) * y.sc.y;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) s[r] = __builtin_fmaf(y.sc.x, s[r], y.k[r] * delta);
+        if (o && kg == 0 && live) *o = __builtin_fmaf(y.sc.x, qoT, delta * y.sc.z);
+    };
+    // tokens c0 .. c1-1 of the chunk; `o`: their outputs, a row apart
+    auto walk = [&](int c0, int c1, float* o) {
+        if (c0 >= c1) return;
+        const size_t os = o ? lg.valueDim : 0;
+        Tok y, z;
+        fetch(y, c0);
+        int c = c0;
+        for (; c + 2 <= c1; c += 2) {
+            fetch(z, c + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            advance(y, o);
+            fetch(y, min(c + 2, GDN_CH - 1));   // past the last token: read and not used
+            __builtin_amdgcn_sched_barrier(0);
+            advance(z, o ? o + os : nullptr);
+            o += 2 * os;
+        }
+        if (c < c1) advance(y, o);
+    };
+    load(0);
+    for (int t0 = 0; t0 < total; t0 += GDN_CH) {
+        prepare(t0);
+        __syncthreads();
+        if (t0 + GDN_CH < total) load(t0 + GDN_CH);   // in flight under the walk
+        const int nt = min(GDN_CH, total - t0);
+        int c0 = 0;
+        if (t0 == 0) {   // the kept rows are all in the first chunk
+            c0 = keep;
+            walk(0, c0, nullptr);
+            if (jb.snap) put_state(Ssnap);
+        }
+        walk(c0, nt, core + (size_t)(jb.row0 + t0 + c0 - keep) * lg.valueDim + h * lg.Dv + vv);
+        __syncthreads();   // the chunk's LDS is free
+    }
+    put_state(S);
+}
+
+template <int DK>
+static void launch_gdn_dk(hipStream_t st, const float* lraw, const float* lrep, int njobs, const JobDev* jobs,
+                          const float* gp, const LinGeom& lg, float* state, float* core, int longest) {
+    const dim3 grid((lg.Dv + GDN_TV - 1) / GDN_TV, lg.nV, njobs), blk(GDN_T);
+    if (longest <= GDN_FEW)
+        hipLaunchKernelGGL(k_gdn_few<DK>, grid, blk, 0, st, lraw, lrep, jobs, gp, lg, state, core);
+    else
+        hipLaunchKernelGGL(k_gdn<DK>, grid, blk, 0, st, lraw, lrep, jobs, gp, lg, state, core);
+}
+
 void launch_gdn(hipStream_t st, const float* lraw, const float* lrep, int njobs, const JobDev* jobs, const float* gp,
-                const LinGeom& lg, float* state, float* core) {
+                const LinGeom& lg, float* state, float* core, int longest) {
     if (njobs <= 0) return;
-    const dim3 grid((lg.Dv + GDN_TV - 1) / GDN_TV, lg.nV, njobs), blk(GDN_KS * GDN_TV);
     switch (lg.Dk) {
-        case 16: hipLaunchKernelGGL(k_gdn<16>, grid, blk, 0, st, lraw, lrep, jobs, gp, lg, state, core); break;
-        case 32: hipLaunchKernelGGL(k_gdn<32>, grid, blk, 0, st, lraw, lrep, jobs, gp, lg, state, core); break;
-        case 64: hipLaunchKernelGGL(k_gdn<64>, grid, blk, 0, st, lraw, lrep, jobs, gp, lg, state, core); break;
-        default: hipLaunchKernelGGL(k_gdn<128>, grid, blk, 0, st, lraw, lrep, jobs, gp, lg, state, core); break;
+        case 16: launch_gdn_dk<16>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, longest); break;
+        case 32: launch_gdn_dk<32>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, longest); break;
+        case 64: launch_gdn_dk<64>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, longest); break;
+        default: launch_gdn_dk<128>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, longest); break;
     }
     CHECK_LAUNCH();
 }
