@@ -46,6 +46,10 @@ struct Layer {
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 constexpr int MTP_STEPS_MAX = 7;   // SPEC_COLS - 1 drafts (stage.js:303-304)
+// f16 rows cross between the caller's memory, pinned memory and the device in
+// pieces of this many bytes (results: at most IO_PIECES_MAX of them).
+constexpr size_t IO_PIECE = (size_t)1 << 20;
+constexpr int IO_PIECES_MAX = 16;
 constexpr int PPW_NARROW = 2;   // pages per attention item for narrow K/V rows (nKV * D <= 512)
 
 }  // namespace
@@ -123,20 +127,19 @@ struct cc_ctx {
     uint64_t* tk_a = nullptr;
     uint64_t* tk_scratch = nullptr;   // this device's static scratch (cc_topk_noalloc)
     uint64_t* tk_b = nullptr;
-    float* d_vals = nullptr;
-    uint32_t* d_ids = nullptr;
+    float* d_vals = nullptr;       // a pass's candidates, then (after its values) their ids
     // cc_decode_steps' per-step outputs, grown to the largest call
     float* dec_vals = nullptr;
     uint32_t* dec_ids = nullptr;
     size_t dec_cap = 0;
     int32_t* dec_plan = nullptr;   // cc_decode_steps: every pass's page pops
     size_t dec_plan_cap = 0;       // (int32 entries)
-    uint16_t* d_hbits = nullptr;
     // per-step metadata (device) and its pinned host staging
     uint8_t* d_meta = nullptr;
     uint8_t* h_meta = nullptr;
     size_t meta_bytes = 0;
-    void* h_out = nullptr;
+    void* h_out = nullptr;         // results, pinned: kernels write them here
+    std::vector<hipEvent_t> out_ev;   // one a piece of a large pass's rows
     size_t out_bytes = 0;
     hipStream_t stream = nullptr;
     std::string err;
@@ -317,12 +320,14 @@ struct StepPlan {
 };
 
 // Per-step metadata. First what the host writes each pass (the page plan,
-// the jobs for the device packer, ids | hidden rows, the MTP fill's rows),
-// copied in one transfer; then what the device packer builds (jobs, items,
-// row_job, head_rows, combine workgroups (job, kv head, m-tile)).
+// the jobs for the device packer, ids, the MTP fill's rows), the first
+// `jobs` bytes, copied in one go; then what the device packer builds (jobs,
+// items, row_job, head_rows, combine workgroups (job, kv head, m-tile)).
+// The host's copy has the f16 rows handed in after all that, at `hidden`
+// (kernels read them where they are).
 struct MetaLayout {
-    size_t plan, pack, ids, mtp_jobs, mtp_row_job, mtp_src, mtp_ids, hidden;
-    size_t jobs, items, row_job, head_rows, cwg, total;
+    size_t plan, pack, ids, mtp_jobs, mtp_row_job, mtp_src, mtp_ids;
+    size_t jobs, items, row_job, head_rows, cwg, total, hidden;
 };
 
 // (job, kv head, m-tile) triples a pass can hold.
@@ -331,7 +336,7 @@ size_t max_cwg_for(const cc_ctx* ctx) {
 }
 
 MetaLayout meta_layout(const cc_ctx* ctx) {
-    const int max_jobs = ctx->o.max_jobs, t_max = ctx->o.t_max, H = ctx->d.hidden;
+    const int max_jobs = ctx->o.max_jobs, t_max = ctx->o.t_max;
     MetaLayout m{};
     size_t at = 0;
     auto take = [&](size_t bytes) { size_t r = at; at += (bytes + 255) & ~(size_t)255; return r; };
@@ -344,13 +349,12 @@ MetaLayout meta_layout(const cc_ctx* ctx) {
     m.mtp_row_job = take(4 * (size_t)t_max);
     m.mtp_src = take(4 * (size_t)t_max);
     m.mtp_ids = take(4 * (size_t)t_max);
-    m.hidden = take(2 * (size_t)t_max * H);
     m.jobs = take(sizeof(JobDev) * max_jobs);
     m.items = take(sizeof(AttnItem) * ctx->items_cap);
     m.row_job = take(4 * (size_t)t_max);
     m.head_rows = take(4 * (size_t)t_max);
     m.cwg = take(12 * max_cwg_for(ctx));
-    m.total = at;
+    m.total = m.hidden = at;
     return m;
 }
 
@@ -411,6 +415,7 @@ void cc_destroy(cc_ctx* ctx) {
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     for (hipEvent_t e : ctx->pev) (void)hipEventDestroy(e);
+    for (hipEvent_t e : ctx->out_ev) (void)hipEventDestroy(e);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -652,16 +657,15 @@ cc_status cc_create(const cc_dims* dims, const cc_opts* opts, cc_ctx** out) {
             const size_t keys = (size_t)T * ceil_div(d.vocab, 4096) * TOPK_MAX;
             HIPCHK(dalloc(ctx, &ctx->tk_a, keys * 8, &ctx->scratch_bytes));
             HIPCHK(dalloc(ctx, &ctx->tk_b, keys * 8, &ctx->scratch_bytes));
-            HIPCHK(dalloc(ctx, &ctx->d_vals, (size_t)T * TOPK_MAX * 4, &ctx->scratch_bytes));
-            HIPCHK(dalloc(ctx, &ctx->d_ids, (size_t)T * TOPK_MAX * 4, &ctx->scratch_bytes));
+            HIPCHK(dalloc(ctx, &ctx->d_vals, (size_t)T * TOPK_MAX * 8 + 16, &ctx->scratch_bytes));
         }
-        HIPCHK(dalloc(ctx, &ctx->d_hbits, (size_t)T * H * 2, &ctx->scratch_bytes));
         MetaLayout ml = meta_layout(ctx);
         ctx->meta_bytes = ml.total;
         HIPCHK(dalloc(ctx, &ctx->d_meta, ml.total, &ctx->scratch_bytes));
-        HIPCHK(hipHostMalloc((void**)&ctx->h_meta, ml.total, hipHostMallocDefault));
+        // coherent: kernels read and write it while the host does, pass after pass
+        HIPCHK(hipHostMalloc((void**)&ctx->h_meta, ml.hidden + (size_t)T * H * 2, hipHostMallocCoherent));
         ctx->out_bytes = std::max((size_t)T * TOPK_MAX * 8, (size_t)T * H * 2) + 256;
-        HIPCHK(hipHostMalloc(&ctx->h_out, ctx->out_bytes, hipHostMallocDefault));
+        HIPCHK(hipHostMalloc(&ctx->h_out, ctx->out_bytes, hipHostMallocCoherent));
         HIPCHK(hipStreamSynchronize(ctx->stream));
         return CC_OK;
     };
@@ -1313,7 +1317,7 @@ static void mtp_input(cc_ctx* ctx, const int32_t* ids, float* hin, int T) {
     const cc_dims& d = ctx->d;
     hipStream_t st = ctx->stream;
     const int H = d.hidden, KUH = ceil_div(H, 64), Mpad = mpad_of(T);
-    launch_embed(st, ids, nullptr, T, ctx->embed_draft, ctx->mtp_e, 0);
+    launch_embed(st, ids, T, ctx->embed_draft, ctx->mtp_e, 0);
     launch_resid_norm(st, ctx->mtp_e, nullptr, nullptr, 0, T, Mpad, H, 0, ctx->enorm, d.rms_eps, KUH, ctx->xp_e,
                       nullptr);
     launch_resid_norm(st, hin, nullptr, nullptr, 0, T, Mpad, H, 0, ctx->hnorm, d.rms_eps, KUH, ctx->xp_hh, nullptr);
@@ -1513,7 +1517,6 @@ cc_status cc_step(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_t at, in
             total += nw;
         }
     }
-    size_t copy_bytes = ml.hidden;
     // The MTP jobs' rows, packed (stage.js:1404-1421): row 0 of a job pairs
     // its first token with the session's kept row, row i with the job's row
     // i - 1.
@@ -1544,18 +1547,10 @@ cc_status cc_step(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_t at, in
         int r = 0;
         for (int j = 0; j < njobs; j++)
             for (int i = 0; i < jobs[j].n; i++) ids[r++] = jobs[j].ids[i];
-    } else {
-        uint16_t* hid = (uint16_t*)(hm + ml.hidden);
-        size_t r = 0;
-        for (int j = 0; j < njobs; j++) {
-            std::memcpy(hid + r, jobs[j].hidden, (size_t)jobs[j].n * d.hidden * 2);
-            r += (size_t)jobs[j].n * d.hidden;
-        }
-        copy_bytes = ml.hidden + (size_t)T * d.hidden * 2;
     }
     hipStream_t st = ctx->stream;
     HIPCHK(hipEventRecord(ctx->ev0, st));
-    HIPCHK(hipMemcpyAsync(ctx->d_meta, hm, copy_bytes, hipMemcpyHostToDevice, st));
+    launch_copy16(st, hm, ctx->d_meta, ml.jobs);
     pack_on_device(ctx, ml, njobs, p.nlaunch, 0, head);
     cc_status ps = take_pages(ctx, want, (int32_t*)(ctx->d_meta + ml.plan), (int32_t*)(hm + ml.plan), status);
     if (ps != CC_OK) {
@@ -1565,15 +1560,30 @@ cc_status cc_step(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_t at, in
     // Embedding (position 0) or the rows handed in.
     QTensor emb = ctx->wte;
     emb.K = d.hidden;
-    if (gather) launch_embed(st, (const int32_t*)(ctx->d_meta + ml.ids), nullptr, T, emb, ctx->x);
+    if (gather) launch_embed(st, (const int32_t*)(ctx->d_meta + ml.ids), T, emb, ctx->x);
     else {
-        QTensor shape;
-        shape.K = d.hidden;
-        launch_embed(st, nullptr, (const uint16_t*)(ctx->d_meta + ml.hidden), T, shape, ctx->x);
+        // the rows into pinned memory, and from there to the device a piece at
+        // a time, so the link works while the host copies the next piece
+        uint16_t* hid = (uint16_t*)(hm + ml.hidden);
+        const size_t H = d.hidden;
+        const int piece = (int)std::max<size_t>(1, IO_PIECE / (H * 2));
+        int r = 0, sent = 0;
+        for (int j = 0; j < njobs; j++)
+            for (int i = 0; i < jobs[j].n;) {
+                const int n = std::min(jobs[j].n - i, sent + piece - r);
+                std::memcpy(hid + r * H, jobs[j].hidden + i * H, (size_t)n * H * 2);
+                i += n;
+                r += n;
+                if (r == sent + piece || r == T) {
+                    launch_rows_in(st, hid + sent * H, (int64_t)(r - sent) * H, ctx->x + sent * H);
+                    sent = r;
+                }
+            }
     }
     const int b0 = std::max(at, 1) - 1, b1 = std::min(to, d.n_layer + 1) - 1;
     if (b1 > b0) run_blocks(ctx, p, ml, b0, b1);
     void* hout = ctx->h_out;
+    std::vector<int64_t> out_at;   // where the pieces of the rows begin, and their end
     if (head) {
         const QTensor& hw = d.tied ? ctx->wte : ctx->lm_head;
         const int S = p.S;
@@ -1582,13 +1592,28 @@ cc_status cc_step(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_t at, in
                           ctx->norm, d.rms_eps, hw.KU, ctx->xp_h, nullptr);
         launch_gemm(st, hw, ctx->xp_h, ctx->mt_alloc, ctx->logits, S, ctx->ncu);
         ctx->head_rows = S;
-        launch_topk(st, ctx->logits, gemm_planes(hw, S, ctx->ncu), S, d.vocab, topk, ctx->tk_a, ctx->tk_b, ctx->d_vals, ctx->d_ids);
-        HIPCHK(hipMemcpyAsync(hout, ctx->d_vals, (size_t)S * topk * 4, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync((uint8_t*)hout + (size_t)S * topk * 4, ctx->d_ids, (size_t)S * topk * 4,
-                              hipMemcpyDeviceToHost, st));
+        launch_topk(st, ctx->logits, gemm_planes(hw, S, ctx->ncu), S, d.vocab, topk, ctx->tk_a, ctx->tk_b, ctx->d_vals,
+                    (uint32_t*)(ctx->d_vals + (size_t)S * topk));
+        launch_copy16(st, ctx->d_vals, hout, (size_t)S * topk * 8);
     } else if (!at_end) {
-        launch_to_half_bits(st, ctx->x, (int64_t)T * d.hidden, ctx->d_hbits);
-        HIPCHK(hipMemcpyAsync(hout, ctx->d_hbits, (size_t)T * d.hidden * 2, hipMemcpyDeviceToHost, st));
+        // straight into pinned memory; a large pass in pieces, each copied out
+        // below while the next one crosses the link
+        const int64_t n = (int64_t)T * d.hidden;
+        const int pieces = (int)std::min<int64_t>(IO_PIECES_MAX, std::max<int64_t>(1, n * 2 / IO_PIECE));
+        const int64_t step = (n / 8 + pieces - 1) / pieces * 8;
+        for (int64_t at8 = 0; at8 < n; at8 += step) {
+            launch_to_half_bits(st, ctx->x + at8, std::min(step, n - at8), (uint16_t*)hout + at8);
+            if (pieces == 1) break;
+            const size_t k = out_at.size();
+            if (ctx->out_ev.size() == k) {
+                hipEvent_t e;
+                HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+                ctx->out_ev.push_back(e);
+            }
+            HIPCHK(hipEventRecord(ctx->out_ev[k], st));
+            out_at.push_back(at8);
+        }
+        if (pieces > 1) out_at.push_back(n);
     }
     if (Tm > 0) {
         mtp_fill(ctx, ml, Tm, nmj);
@@ -1602,6 +1627,10 @@ cc_status cc_step(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_t at, in
     }
     HIPCHK(hipEventRecord(ctx->ev1, st));
     if (ctx->prof) prof_replay(ctx, p, ml, b0, b1, head);
+    for (size_t k = 0; k + 1 < out_at.size(); k++) {
+        HIPCHK(hipEventSynchronize(ctx->out_ev[k]));
+        std::memcpy(hidden_out + out_at[k], (const uint16_t*)hout + out_at[k], (size_t)(out_at[k + 1] - out_at[k]) * 2);
+    }
     HIPCHK(hipStreamSynchronize(st));
     HIPCHK(take_launch_error());
     float ms = 0;
@@ -1627,7 +1656,7 @@ cc_status cc_step(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_t at, in
     if (head) {
         std::memcpy(top_vals, hout, (size_t)p.S * topk * 4);
         std::memcpy(top_ids, (uint8_t*)hout + (size_t)p.S * topk * 4, (size_t)p.S * topk * 4);
-    } else if (!at_end) {
+    } else if (!at_end && out_at.empty()) {
         std::memcpy(hidden_out, hout, (size_t)T * d.hidden * 2);
     }
     return CC_OK;
@@ -1734,7 +1763,7 @@ cc_status cc_decode_steps(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_
     }
     hipStream_t st = ctx->stream;
     HIPCHK(hipEventRecord(ctx->ev0, st));
-    HIPCHK(hipMemcpyAsync(ctx->d_meta, hm, ml.hidden, hipMemcpyHostToDevice, st));
+    HIPCHK(hipMemcpyAsync(ctx->d_meta, hm, ml.jobs, hipMemcpyHostToDevice, st));
     if (!pplan.empty())
         HIPCHK(hipMemcpyAsync(ctx->dec_plan, pplan.data(), pplan.size() * 4, hipMemcpyHostToDevice, st));
     const QTensor& hw = d.tied ? ctx->wte : ctx->lm_head;
@@ -1751,7 +1780,7 @@ cc_status cc_decode_steps(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_
         plan_jobs(ctx, cur.data(), njobs, p, true);
         pack_on_device(ctx, ml, njobs, p.nlaunch, k, true);
         if (k > 0) launch_ids_col0(st, ctx->dec_ids + (k - 1) * per, S, topk, d_ids_in);
-        launch_embed(st, d_ids_in, nullptr, p.T, emb, ctx->x);
+        launch_embed(st, d_ids_in, p.T, emb, ctx->x);
         run_blocks(ctx, p, ml, 0, d.n_layer);
         launch_resid_norm(st, ctx->x, (const int32_t*)(ctx->d_meta + ml.head_rows), nullptr, 0, S, Mpad, d.hidden, 0,
                           ctx->norm, d.rms_eps, hw.KU, ctx->xp_h, nullptr);

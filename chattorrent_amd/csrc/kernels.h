@@ -157,8 +157,7 @@ void launch_lin_norm(hipStream_t st, const float* core, const float* lraw, const
                      int M, const LinGeom& lg, int KU, uint4* Xp);
 // round: the trunk's rows are rounded to f16 (stage.js:1365-1370); the MTP
 // head's draft embedding is not (model.js:545). An id past wte.N reads zero.
-void launch_embed(hipStream_t st, const int32_t* ids, const uint16_t* hidden, int T, const QTensor& wte,
-                  float* x, int round = 1);
+void launch_embed(hipStream_t st, const int32_t* ids, int T, const QTensor& wte, float* x, int round = 1);
 void launch_gather_rows(hipStream_t st, const float* x, const float* alt, const int32_t* src, int T, int H,
                         float* rows);
 void launch_topk(hipStream_t st, const float* logits, int planes, int rows, int V, int M, uint64_t* a,
@@ -226,4 +225,8 @@ void launch_attn_combine(hipStream_t st, const JobDev* jobs, const float* part, 
                          int KU, uint4* Xp, float* ctx_out, const int32_t* wg_job, int nwg,
                          const float* gate = nullptr);
 void launch_sum_splits(hipStream_t st, const float* part, int splits, int M, int N, float* out);
+// Between the device and the context's pinned host memory, inside kernels:
+// `bytes` rounded up to 16; n values, a multiple of 8.
+void launch_copy16(hipStream_t st, const void* src, void* dst, size_t bytes);
+void launch_rows_in(hipStream_t st, const uint16_t* hidden, int64_t n, float* x);
 void launch_to_half_bits(hipStream_t st, const float* x, int64_t n, uint16_t* out);

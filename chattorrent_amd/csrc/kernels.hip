@@ -3050,18 +3050,12 @@ void launch_attn_combine(hipStream_t st, const JobDev* jobs, const float* part, 
 
 // =============================================================== embedding ===
 // gather_embed_nopos_q8 (web/model/kernels.js:895-917) + round_f16 (the
-// embedding rows are rounded like a block's output, stage.js:1365-1370);
-// or, for a pass entering past position 0, the f16 rows handed in.
-__global__ void k_embed(const int32_t* __restrict__ ids, const uint16_t* __restrict__ hidden, int T, int H,
-                        const uint8_t* __restrict__ rec, int Nt, int KU, int P, int f32s, float* __restrict__ x,
-                        int round, int nrows) {
+// embedding rows are rounded like a block's output, stage.js:1365-1370).
+__global__ void k_embed(const int32_t* __restrict__ ids, int T, int H, const uint8_t* __restrict__ rec, int Nt, int KU, int P,
+                        int f32s, float* __restrict__ x, int round, int nrows) {
     const int t = blockIdx.y;
     const int h = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= T || h >= H) return;
-    if (!ids) {
-        x[(size_t)t * H + h] = half_value(hidden[(size_t)t * H + h]);
-        return;
-    }
     const int v = ids[t];
     if (v < 0 || v >= nrows) {   // a token outside a shorter table (the MTP's draft rows) reads zero
         x[(size_t)t * H + h] = 0.0f;
@@ -3077,11 +3071,10 @@ __global__ void k_embed(const int32_t* __restrict__ ids, const uint16_t* __restr
     x[(size_t)t * H + h] = round ? round_f16_value(e) : e;
 }
 
-void launch_embed(hipStream_t st, const int32_t* ids, const uint16_t* hidden, int T, const QTensor& wte,
-                  float* x, int round) {
+void launch_embed(hipStream_t st, const int32_t* ids, int T, const QTensor& wte, float* x, int round) {
     dim3 grid((wte.K + 255) / 256, T);
-    hipLaunchKernelGGL(k_embed, grid, dim3(256), 0, st, ids, hidden, T, wte.K, wte.codes, wte.Nt, wte.KU, wte.P,
-                       wte.f32s, x, round, ids ? wte.N : 0);
+    hipLaunchKernelGGL(k_embed, grid, dim3(256), 0, st, ids, T, wte.K, wte.codes, wte.Nt, wte.KU, wte.P, wte.f32s, x,
+                       round, wte.N);
     CHECK_LAUNCH();
 }
 
@@ -3846,16 +3839,59 @@ void launch_sum_splits(hipStream_t st, const float* part, int splits, int M, int
     CHECK_LAUNCH();
 }
 
-// Rows of f16 values kept as f32 -> their half bits (exact).
-__global__ void k_to_half_bits(const float* __restrict__ x, int64_t n, uint16_t* __restrict__ out) {
+// ------------------------------------------------ to and from the host ---
+// A pass's small tables, its f16 rows and its results cross the link inside
+// kernels that read or write the context's pinned host memory 16 bytes a
+// thread, each byte once: a copy on its own waits for the copy engine and
+// hands over between queues, about 10 us each way, which a pass of one block
+// (150 us of kernels) pays twice.
+__global__ void k_copy16(const uint4* __restrict__ src, uint4* __restrict__ dst, int64_t n) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = half_bits(x[i]);
+        dst[i] = src[i];
+}
+
+void launch_copy16(hipStream_t st, const void* src, void* dst, size_t bytes) {
+    const int64_t n = (int64_t)((bytes + 15) / 16);
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_copy16, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 65536)), dim3(256), 0, st,
+                       (const uint4*)src, (uint4*)dst, n);
+    CHECK_LAUNCH();
+}
+
+// The f16 rows a pass past position 0 is handed, as f32, 8 values a thread.
+__global__ void k_rows_in(const uint4* __restrict__ hidden, int64_t n8, float4* __restrict__ x) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n8; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint4 q = hidden[i];
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = half_value((uint16_t)(w[e >> 1] >> (16 * (e & 1))));
+        x[2 * i] = make_float4(v[0], v[1], v[2], v[3]);
+        x[2 * i + 1] = make_float4(v[4], v[5], v[6], v[7]);
+    }
+}
+
+void launch_rows_in(hipStream_t st, const uint16_t* hidden, int64_t n, float* x) {
+    if (n <= 0) return;
+    const int64_t n8 = n / 8;
+    hipLaunchKernelGGL(k_rows_in, dim3((unsigned)std::min<int64_t>((n8 + 255) / 256, 65536)), dim3(256), 0, st,
+                       (const uint4*)hidden, n8, (float4*)x);
+    CHECK_LAUNCH();
+}
+
+// Rows of f16 values kept as f32 -> their half bits (exact), 8 values a thread.
+__global__ void k_to_half_bits(const float4* __restrict__ x, int64_t n8, uint4* __restrict__ out) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n8; i += (int64_t)gridDim.x * blockDim.x) {
+        const float4 a = x[2 * i], b = x[2 * i + 1];
+        out[i] = make_uint4(half_bits(a.x) | (uint32_t)half_bits(a.y) << 16, half_bits(a.z) | (uint32_t)half_bits(a.w) << 16,
+                            half_bits(b.x) | (uint32_t)half_bits(b.y) << 16, half_bits(b.z) | (uint32_t)half_bits(b.w) << 16);
+    }
 }
 
 void launch_to_half_bits(hipStream_t st, const float* x, int64_t n, uint16_t* out) {
-    int64_t blocks = (n + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_to_half_bits, dim3((unsigned)blocks), dim3(256), 0, st, x, n, out);
+    if (n <= 0) return;
+    const int64_t n8 = n / 8;
+    hipLaunchKernelGGL(k_to_half_bits, dim3((unsigned)std::min<int64_t>((n8 + 255) / 256, 65536)), dim3(256), 0, st,
+                       (const float4*)x, n8, (uint4*)out);
     CHECK_LAUNCH();
 }

@@ -236,6 +236,31 @@ def test_packed_by_many_workgroups_equals_alone(gpu, njobs, longest, nverify):
         c.close()
 
 
+@pytest.mark.parametrize("rows", [(1,), (127,), (128, 129), (300, 277)])
+def test_rows_in_and_out_in_pieces(gpu, rows):
+    """f16 rows cross to and from the device in 1 MB pieces (128 rows of 4096
+    here): passes of one piece, at its edge, and of several with jobs cut
+    inside a piece return every row as passes of 40 rows do, bit for bit."""
+    from chattorrent_amd.ccdecode import Context
+    rng = np.random.default_rng(sum(rows))
+    d = configs.with_layers(configs.LLAMA8B, 1)
+    c = Context(d, n_max=320, t_max=sum(rows), slots=len(rows), lo=1, hi=2)
+    try:
+        c.fill_random(SEED)
+        hid = [rng.standard_normal((n, d["hidden"])).astype(np.float16).view(np.uint16) for n in rows]
+        for _ in range(2):        # the second pass reuses the pinned memory
+            got = c.step([dict(slot=s, past=0, n=n, hidden=hid[s]) for s, n in enumerate(rows)], at=1, to=2)
+        at = 0
+        for s, n in enumerate(rows):
+            for a in range(0, n, 40):
+                b = min(n, a + 40)
+                part = c.step([dict(slot=s, past=a, n=b - a, hidden=hid[s][a:b])], at=1, to=2)
+                assert np.array_equal(part, got[at + a:at + b]), (s, a)
+            at += n
+    finally:
+        c.close()
+
+
 def test_verify_rows_equal_one_row_jobs(smol):
     """docs/model.md 'Matching plain decoding row by row': row i of an 8-row
     verify gives the bits of a one-row job at past + i."""
