@@ -113,6 +113,8 @@ struct cc_ctx {
     float* ssp = nullptr;          // rmsnorm partial sums of squares [rows][RW_SMAX]
     float* part = nullptr;
     size_t part_floats = 0;
+    float* x2 = nullptr;           // second buffers of a pass of few rows (run_blocks)
+    float* part2 = nullptr;
     int ncu = 0;                   // compute units: the matmul's workgroup count
     uint4* qp = nullptr;
     size_t qp_units = 0;
@@ -592,6 +594,10 @@ cc_status cc_create(const cc_dims* dims, const cc_opts* opts, cc_ctx** out) {
                 if (q->codes) pf = std::max(pf, (size_t)q->P * T * q->N);
         ctx->part_floats = pf;
         HIPCHK(dalloc(ctx, &ctx->part, pf * 4, &ctx->scratch_bytes));
+        // gemm_fuses' second buffers, for its rows
+        const int Tf = std::min(T, GEMM_FUSE_ROWS);
+        HIPCHK(dalloc(ctx, &ctx->x2, (size_t)Tf * H * 4, &ctx->scratch_bytes));
+        HIPCHK(dalloc(ctx, &ctx->part2, pf / T * Tf * 4 + 64, &ctx->scratch_bytes));
         // Q operands: sum over jobs of nKV * ceil(n*group/16) * ng * 2 * 64 uint4.
         ctx->qp_units = (size_t)(ceil_div(T * ctx->group, 16) + o.max_jobs) * nKV * (D / 32) * 128;
         HIPCHK(dalloc(ctx, &ctx->qp, ctx->qp_units * 16, &ctx->scratch_bytes));
@@ -1211,16 +1217,14 @@ static RowScale row_scale_of(const cc_ctx* ctx) {
     return rs;
 }
 
-// fullBlockSegs's attention half (model.js:368-410) on rows x [T][H] whose
-// operand x*ln1 and sums of squares are in place: q|k|v (+ attn_gate) GEMM,
-// finish (row factor, q/k norm, RoPE, KV store, Q operand), attention,
-// combine (output gate, o_proj operand), o GEMM, residual with the operand
-// x*ln2 for the MLP.
-static void full_attn_half(cc_ctx* ctx, Layer& L, float* x, int T, int Mpad, const PassMeta& pm) {
+// fullBlockSegs's attention half (model.js:368-410) between its q|k|v (+
+// attn_gate) planes and o_proj's, both in `part`: finish (row factor, q/k
+// norm, RoPE, KV store, Q operand), attention, combine (output gate, o_proj
+// operand), o GEMM.
+static void attn_mid(cc_ctx* ctx, Layer& L, float* part, int T, const PassMeta& pm) {
     const cc_dims& d = ctx->d;
     hipStream_t st = ctx->stream;
-    const int H = d.hidden, nH = d.n_heads;
-    const RowScale rs = row_scale_of(ctx);
+    const int nH = d.n_heads;
     QkExtras ex;
     if (ctx->hybrid) {
         ex.qn = L.qn;
@@ -1228,30 +1232,35 @@ static void full_attn_half(cc_ctx* ctx, Layer& L, float* x, int T, int Mpad, con
         ex.eps = d.rms_eps;
         ex.gate = ctx->gbuf;
     }
-    launch_gemm(st, L.qkv, ctx->xp_h, ctx->mt_alloc, ctx->part, T, ctx->ncu);
-    launch_fin_qkv(st, ctx->part, gemm_planes(L.qkv, T, ctx->ncu), T, pm.row_job, pm.jobs, nH, ctx->group, ctx->geom, ctx->tbl, ctx->rot,
-                   L.kpool, L.vpool, ctx->page_table, ctx->qp, rs, 1, 1, ex);
+    launch_fin_qkv(st, part, gemm_planes(L.qkv, T, ctx->ncu), T, pm.row_job, pm.jobs, nH, ctx->group, ctx->geom, ctx->tbl, ctx->rot,
+                   L.kpool, L.vpool, ctx->page_table, ctx->qp, row_scale_of(ctx), 1, 1, ex);
     launch_attn(st, pm.items, pm.nlaunch, ctx->qp, L.kpool, L.vpool, ctx->page_table, ctx->geom, ctx->group,
                 ctx->ppw, ctx->apart, pm.multi, ctx->attn);
     launch_attn_combine(st, pm.jobs, ctx->apart, ctx->geom, nH, ctx->group, L.o.KU, ctx->xp_o, nullptr, pm.cwg,
                         pm.ncwg, ctx->hybrid ? ctx->gbuf : nullptr);
-    launch_gemm(st, L.o, ctx->xp_o, ctx->mt_alloc, ctx->part, T, ctx->ncu);
-    launch_resid_w(st, x, ctx->part, gemm_planes(L.o, T, ctx->ncu), T, Mpad, H, 0, L.ln2, ceil_div(H, 64), ctx->xp_h, ctx->ssp);
+    launch_gemm(st, L.o, ctx->xp_o, ctx->mt_alloc, part, T, ctx->ncu);
+}
+
+// The attention half on rows x [T][H] whose operand x*ln1 and sums of squares
+// are in place, with the residual and the operand x*ln2 for the MLP.
+static void full_attn_half(cc_ctx* ctx, Layer& L, float* x, int T, int Mpad, const PassMeta& pm) {
+    hipStream_t st = ctx->stream;
+    const int H = ctx->d.hidden;
+    launch_gemm(st, L.qkv, ctx->xp_h, ctx->mt_alloc, ctx->part, T, ctx->ncu);
+    attn_mid(ctx, L, ctx->part, T, pm);
+    launch_resid_w(st, x, x, ctx->part, gemm_planes(L.o, T, ctx->ncu), T, Mpad, H, 0, L.ln2, ceil_div(H, 64), ctx->xp_h, ctx->ssp);
 }
 
 // The SwiGLU MLP (model.js:307-315) from the operand x*ln2: gate|up GEMM,
-// finish (row factor, silu*up), down GEMM, residual (+ round_f16 for a
-// trunk block) and the next block's operand x*next_ln1 (or none).
-static void ffn_half(cc_ctx* ctx, Layer& L, float* x, int T, int Mpad, int round, const float* next_ln1) {
+// finish (row factor, silu*up), down GEMM, residual. The MTP block's; the
+// trunk's blocks are in run_blocks.
+static void ffn_half(cc_ctx* ctx, Layer& L, float* x, int T, int Mpad) {
     const cc_dims& d = ctx->d;
     hipStream_t st = ctx->stream;
-    const int H = d.hidden;
-    const RowScale rs = row_scale_of(ctx);
     launch_gemm(st, L.gu, ctx->xp_h, ctx->mt_alloc, ctx->part, T, ctx->ncu);
-    launch_fin_swiglu(st, ctx->part, gemm_planes(L.gu, T, ctx->ncu), T, Mpad, d.ffn, L.down.KU, ctx->xp_f, rs);
+    launch_fin_swiglu(st, ctx->part, gemm_planes(L.gu, T, ctx->ncu), T, Mpad, d.ffn, L.down.KU, ctx->xp_f, row_scale_of(ctx));
     launch_gemm(st, L.down, ctx->xp_f, ctx->mt_alloc, ctx->part, T, ctx->ncu);
-    launch_resid_w(st, x, ctx->part, gemm_planes(L.down, T, ctx->ncu), T, Mpad, H, round, next_ln1, next_ln1 ? ceil_div(H, 64) : 0,
-                   next_ln1 ? ctx->xp_h : nullptr, ctx->ssp);
+    launch_resid_w(st, x, x, ctx->part, gemm_planes(L.down, T, ctx->ncu), T, Mpad, d.hidden, 0, nullptr, 0, nullptr, ctx->ssp);
 }
 
 static int mpad_of(int T) { return 16 * ceil_div(T, 16) + (ceil_div(T, 16) > 1 && (ceil_div(T, 16) & 1) ? 16 : 0); }
@@ -1283,29 +1292,62 @@ static void run_blocks(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, int
     const int KUH = ceil_div(H, 64);   // every block's first matmul reads K = hidden
     int longest = 0;                   // a long job takes the row-parallel conv
     for (const JobDev& jd : p.jobs) longest = std::max(longest, (int)jd.n);
+    auto planes = [&](const QTensor& w) { return gemm_planes(w, T, ctx->ncu); };
+    // With few rows (gemm_fuses) a matmul adds the planes before it to the
+    // residual rows itself, or forms SwiGLU itself, in place of a launch
+    // between the two: then the rows and the planes move to the other buffer
+    // of their pair, since the matmul's workgroups still read the old ones.
+    float *x = ctx->x, *x2 = ctx->x2, *pa = ctx->part, *pb = ctx->part2;
+    auto gemm = [&](const QTensor& w, const uint4* xp) { launch_gemm(st, w, xp, ctx->mt_alloc, pa, T, ctx->ncu); };
+    auto gemm_resid = [&](const QTensor& w, const QTensor& before, int round, const float* norm) {
+        launch_gemm_resid(st, w, x, x2, pa, planes(before), round, norm, ctx->ssp, pb, T, ctx->ncu);
+        std::swap(x, x2);
+        std::swap(pa, pb);
+    };
+    bool pending = false;   // the last block's down planes wait for this block's first matmul
     for (int b = b0; b < b1; b++) {
         Layer& L = ctx->layers[b - ctx->L0];
-        if (b == b0) launch_resid_w(st, ctx->x, nullptr, 0, T, Mpad, H, 0, L.ln1, KUH, ctx->xp_h, ctx->ssp);
+        const QTensor& w1 = L.kind == CC_LINEAR_ATTENTION ? L.lin : L.qkv;
+        if (b == b0) launch_resid_w(st, x, x, nullptr, 0, T, Mpad, H, 0, L.ln1, KUH, ctx->xp_h, ctx->ssp);
+        if (pending) gemm_resid(w1, ctx->layers[b - 1 - ctx->L0].down, 1, L.ln1);
+        else gemm(w1, ctx->xp_h);
         if (L.kind == CC_LINEAR_ATTENTION) {
             // linearBlockSegs (model.js:472-527): in_proj, conv + ring, the
             // recurrence on each session's state, gated norm, out_proj
             const LinGeom& lg = ctx->lg;
-            launch_gemm(st, L.lin, ctx->xp_h, ctx->mt_alloc, ctx->part, T, ctx->ncu);
             if (longest > LIN_SEQ_ROWS)
-                launch_lin_conv_rows(st, ctx->part, gemm_planes(L.lin, T, ctx->ncu), T, pm.njobs, pm.row_job, pm.jobs, rs, L.conv, lg, L.state,
+                launch_lin_conv_rows(st, pa, planes(L.lin), T, pm.njobs, pm.row_job, pm.jobs, rs, L.conv, lg, L.state,
                                      ctx->lraw, ctx->lrep, ctx->lring);
             else
-                launch_lin_conv(st, ctx->part, gemm_planes(L.lin, T, ctx->ncu), T, pm.njobs, pm.jobs, rs, L.conv, lg, L.state, ctx->lraw,
+                launch_lin_conv(st, pa, planes(L.lin), T, pm.njobs, pm.jobs, rs, L.conv, lg, L.state, ctx->lraw,
                                 ctx->lrep);
             launch_gdn(st, ctx->lraw, ctx->lrep, pm.njobs, pm.jobs, L.gp, lg, L.state, ctx->lcore, longest);
             launch_lin_norm(st, ctx->lcore, ctx->lraw, L.gnorm, d.rms_eps, T, lg, L.out.KU, ctx->xp_v);
-            launch_gemm(st, L.out, ctx->xp_v, ctx->mt_alloc, ctx->part, T, ctx->ncu);
-            launch_resid_w(st, ctx->x, ctx->part, gemm_planes(L.out, T, ctx->ncu), T, Mpad, H, 0, L.ln2, KUH, ctx->xp_h, ctx->ssp);
+            gemm(L.out, ctx->xp_v);
         } else {
-            full_attn_half(ctx, L, ctx->x, T, Mpad, pm);
+            attn_mid(ctx, L, pa, T, pm);
         }
-        const bool next = b + 1 < b1;
-        ffn_half(ctx, L, ctx->x, T, Mpad, 1, next ? ctx->layers[b + 1 - ctx->L0].ln1 : nullptr);
+        const QTensor& w2 = L.kind == CC_LINEAR_ATTENTION ? L.out : L.o;
+        if (gemm_fuses(L.gu, T, planes(w2) + 1)) gemm_resid(L.gu, w2, 0, L.ln2);
+        else {
+            launch_resid_w(st, x, x, pa, planes(w2), T, Mpad, H, 0, L.ln2, KUH, ctx->xp_h, ctx->ssp);
+            gemm(L.gu, ctx->xp_h);
+        }
+        if (gemm_fuses(L.down, T, 2 * planes(L.gu))) {
+            launch_gemm_swiglu(st, L.down, pa, planes(L.gu), d.ffn, rs, pb, T, ctx->ncu);
+            std::swap(pa, pb);
+        } else {
+            launch_fin_swiglu(st, pa, planes(L.gu), T, Mpad, d.ffn, L.down.KU, ctx->xp_f, rs);
+            gemm(L.down, ctx->xp_f);
+        }
+        pending = false;
+        if (b + 1 < b1) {
+            const Layer& Ln = ctx->layers[b + 1 - ctx->L0];
+            pending = gemm_fuses(Ln.kind == CC_LINEAR_ATTENTION ? Ln.lin : Ln.qkv, T, planes(L.down) + 1);
+            if (!pending) launch_resid_w(st, x, x, pa, planes(L.down), T, Mpad, H, 1, Ln.ln1, KUH, ctx->xp_h, ctx->ssp);
+        } else {
+            launch_resid_w(st, x, ctx->x, pa, planes(L.down), T, Mpad, H, 1, nullptr, 0, nullptr, ctx->ssp);
+        }
     }
 }
 
@@ -1324,7 +1366,7 @@ static void mtp_input(cc_ctx* ctx, const int32_t* ids, float* hin, int T) {
     launch_gemm(st, ctx->fc_e, ctx->xp_e, ctx->mt_alloc, ctx->part, T, ctx->ncu);
     launch_sum_splits(st, ctx->part, gemm_planes(ctx->fc_e, T, ctx->ncu), T, H, ctx->mx);
     launch_gemm(st, ctx->fc_h, ctx->xp_hh, ctx->mt_alloc, ctx->part, T, ctx->ncu);
-    launch_resid_w(st, ctx->mx, ctx->part, gemm_planes(ctx->fc_h, T, ctx->ncu), T, Mpad, H, 0, ctx->mtpL.ln1, KUH, ctx->xp_h, ctx->ssp);
+    launch_resid_w(st, ctx->mx, ctx->mx, ctx->part, gemm_planes(ctx->fc_h, T, ctx->ncu), T, Mpad, H, 0, ctx->mtpL.ln1, KUH, ctx->xp_h, ctx->ssp);
 }
 
 // The MTP layer's KV rows for a pass's MTP jobs (stage.js:1404-1421): each
@@ -1888,7 +1930,7 @@ cc_status cc_mtp_draft(cc_ctx* ctx, int32_t slot, int32_t row, int32_t token, in
         pm.ncwg = plans[k].ncwg;
         mtp_input(ctx, ids + k, ctx->mtp_in, 1);
         full_attn_half(ctx, ctx->mtpL, ctx->mx, 1, mpad_of(1), pm);
-        ffn_half(ctx, ctx->mtpL, ctx->mx, 1, mpad_of(1), 0, nullptr);
+        ffn_half(ctx, ctx->mtpL, ctx->mx, 1, mpad_of(1));
         launch_resid_norm(st, ctx->mx, nullptr, nullptr, 0, 1, 32, H, 0, ctx->mtp_norm, d.rms_eps, KUH, ctx->xp_h,
                           nullptr);
         launch_gemm(st, ctx->head_draft, ctx->xp_h, ctx->mt_alloc, ctx->mtp_logits, 1, ctx->ncu);

@@ -203,8 +203,19 @@ hipError_t take_launch_error();
 // Residual step and the next matmul's operand x*w (rmsnorm without its row
 // factor, which the matmul's consumer applies: RowScale), over (slice, row)
 // workgroups; H % 64 == 0. With w null only the residual step runs.
-void launch_resid_w(hipStream_t st, float* x, const float* part, int splits, int M, int Mpad, int H, int round,
-                    const float* w, int KU, uint4* Xp, float* ssp);
+// x + planes go to xo (x itself, or another buffer).
+void launch_resid_w(hipStream_t st, const float* x, float* xo, const float* part, int splits, int M, int Mpad, int H,
+                    int round, const float* w, int KU, uint4* Xp, float* ssp);
+// The matmul with its operand formed by its own workgroups, for few rows:
+// from the residual step (launch_resid_w's, with the new rows in xo, which is
+// not x) or SwiGLU (launch_fin_swiglu's). `part` (the previous projection's
+// planes) and `out` do not overlap. gemm_fuses says for which sizes.
+constexpr int GEMM_FUSE_ROWS = 16;
+bool gemm_fuses(const QTensor& w, int M, int values);
+void launch_gemm_resid(hipStream_t st, const QTensor& w, const float* x, float* xo, const float* part, int splits,
+                       int round, const float* norm, float* ssp, float* out, int M, int ncu);
+void launch_gemm_swiglu(hipStream_t st, const QTensor& w, const float* part, int splits, int F, const RowScale& rs,
+                        float* out, int M, int ncu);
 void launch_resid_norm(hipStream_t st, float* x, const int32_t* rows, const float* part, int splits, int M,
                        int Mpad, int H, int round, const float* w, float eps, int KU, uint4* Xp, float* y);
 // The attention launches of one stream: the CU count and a pair of device

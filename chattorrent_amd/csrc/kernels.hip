@@ -73,12 +73,55 @@ __device__ static inline float rec_scale(uint32_t word, int h) {
     }
 }
 
-template <int MT, bool F32S>
+// Few rows (launch_gemm_resid, launch_gemm_swiglu; gemm_fuses says when): the workgroup forms its
+// plane's operand itself from the previous projection's planes, in place of
+// k_resid_w's or k_fin_swiglu's launch and the operand's way through memory:
+// the same values by the same operations, in as many places as there are
+// column groups. LX_PRO_RESID's grid has workgroups after the matmul's, four
+// (512-column slice, row) pairs each, that store the new residual rows (in
+// another buffer: the others still read the old ones) and the sums of squares.
+// The operand's rows past M stay whatever LDS held: a row of the product
+// depends on its own row alone, and rows past M are not stored.
+// Few rows leave each launch bound by its own start, drain and first loads:
+// three of a block's ten go. One chat: hidden 576, 30 blocks and head
+// 1233 -> 1088 us; hidden 5120, 4 blocks 501 -> 474 us.
+__device__ static inline float row_scale(const RowScale& rs, int m);
+constexpr int LX_PRO_NONE = 0, LX_PRO_RESID = 1, LX_PRO_SWIGLU = 2;
+struct LxPro {
+    const float* part = nullptr;   // the previous projection's planes
+    int splits = 0;
+    const float* x = nullptr;      // RESID: residual rows, the new ones, the norm's weights
+    float* xo = nullptr;
+    const float* w = nullptr;
+    int round = 0;
+    float* ssp = nullptr;
+    int G = 0;                     // the matmul's workgroups
+    RowScale rs;                   // SWIGLU: the row factor
+    int F = 0;
+};
+struct LxNoPro {};
+template <int PRO>
+struct LxProArg { using type = LxPro; };
+template <>
+struct LxProArg<LX_PRO_NONE> { using type = LxNoPro; };   // no prologue, no arguments of one
+template <int N>
+__device__ static inline void resid_row(const LxPro& p, int M, int H, int m, int k0, float (&x)[N]);
+__device__ static inline void swiglu8(const LxPro& p, int M, int m, int k0, float f, float (&v)[8]);
+__device__ static void resid_slices(const LxPro& p, int M, int H, float* red);
+
+template <int MT, bool F32S, int PRO = LX_PRO_NONE>
 __global__ __launch_bounds__(64 * LX_WAVES) void k_gemm_lx(const uint8_t* __restrict__ Wr,
                                                            const uint4* __restrict__ Xp, float* __restrict__ out,
-                                                           int KU, int M, int N, int Nt, int P, int Gm) {
+                                                           int KU, int M, int N, int Nt, int P, int Gm,
+                                                           typename LxProArg<PRO>::type pro) {
+    static_assert(PRO == LX_PRO_NONE || MT == 1, "a prologue forms one m-tile");
     constexpr int NT = 2, R = LX_R, PW = R - 1, WAVES = LX_WAVES;
     extern __shared__ __attribute__((aligned(1024))) u32x4 xs[];
+    if constexpr (PRO == LX_PRO_RESID)
+        if ((int)blockIdx.x >= pro.G) {
+            resid_slices(pro, M, 64 * KU, (float*)xs);
+            return;
+        }
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = blockIdx.x % P, j = blockIdx.x / P;
@@ -115,7 +158,34 @@ __global__ __launch_bounds__(64 * LX_WAVES) void k_gemm_lx(const uint8_t* __rest
         for (int i = 0; i < PW; i++) load_w(w[i], s[i]);
     }
     // Activations of this plane into LDS: block (u, mt, q) of 1 KiB, q = 2h + hl.
-    {
+    if constexpr (PRO != LX_PRO_NONE) {
+        // a thread's 8 columns of a row at a time
+        const int per = 8 * len;
+        for (int i = threadIdx.x; i < M * per; i += 64 * WAVES) {
+            const int m = i / per, c = i % per, k0 = 64 * ua + 8 * c;
+            float v[8];
+            if constexpr (PRO == LX_PRO_RESID) {
+                resid_row<8>(pro, M, 64 * KU, m, k0, v);
+                const float4 wa = *(const float4*)(pro.w + k0), wb = *(const float4*)(pro.w + k0 + 4);
+                const float wv[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = v[e] * wv[e];
+            } else
+                swiglu8(pro, M, m, k0, row_scale(pro.rs, m), v);
+            half8_t hi, lo;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                _Float16 a, b;
+                split_hilo_x(v[e], a, b);
+                hi[e] = a;
+                lo[e] = b;
+            }
+            // unit c / 8, half-group (c % 8) / 4, k-block c % 4
+            u32x4* at = xs + ((c >> 3) * 4 + 2 * ((c >> 2) & 1)) * 64 + m + 16 * (c & 3);
+            at[0] = __builtin_bit_cast(u32x4, hi);
+            at[64] = __builtin_bit_cast(u32x4, lo);
+        }
+    } else {
         const int nblk = len * MT * 4;
         for (int b = wave; b < nblk; b += WAVES) {
             const int u = b / (MT * 4), mt = (b / 4) % MT, q = b % 4;
@@ -291,21 +361,24 @@ int lx_planes_for(int N, int K, int ncu) {
     return P;
 }
 
-template <int MT, bool F32S>
-static void launch_lx(hipStream_t st, const QTensor& w, const uint4* Xp, float* out, int M, int ncu) {
+template <int MT, bool F32S, int PRO = LX_PRO_NONE>
+static void launch_lx(hipStream_t st, const QTensor& w, const uint4* Xp, float* out, int M, int ncu,
+                      typename LxProArg<PRO>::type pro = {}) {
     static bool attr = false;
     if (!attr) {
         attr = true;
-        (void)hipFuncSetAttribute((const void*)k_gemm_lx<MT, F32S>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        (void)hipFuncSetAttribute((const void*)k_gemm_lx<MT, F32S, PRO>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   LX_UNITS * MT * 4096);
     }
     const int G = lx_groups(w, ncu), Gm = G / w.P;
     const int lenmax = (w.KU + w.P - 1) / w.P;
     // the plane's activations, and afterwards the cut parts (1 KiB per wave, m-tile and tile)
     const size_t lds = std::max((size_t)lenmax * MT * 4096, (size_t)LX_WAVES * MT * 2 * 1024);
-    dim3 grid(G, (M + 16 * MT - 1) / (16 * MT));
-    hipLaunchKernelGGL((k_gemm_lx<MT, F32S>), grid, dim3(64 * LX_WAVES), lds, st, (const uint8_t*)w.codes, Xp, out,
-                       w.KU, M, w.N, w.Nt, w.P, Gm);
+    if constexpr (PRO != LX_PRO_NONE) pro.G = G;
+    const int extra = PRO == LX_PRO_RESID ? (M * ((w.K / 4 + RW_THREADS - 1) / RW_THREADS) + 3) / 4 : 0;
+    dim3 grid(G + extra, (M + 16 * MT - 1) / (16 * MT));
+    hipLaunchKernelGGL((k_gemm_lx<MT, F32S, PRO>), grid, dim3(64 * LX_WAVES), lds, st, (const uint8_t*)w.codes, Xp,
+                       out, w.KU, M, w.N, w.Nt, w.P, Gm, pro);
 }
 
 // ------------------------------------------------- many rows (M > 32) ---
@@ -1175,7 +1248,7 @@ __device__ static inline float row_scale(const RowScale& rs, int m) { return row
 // loads are issued at once (4 when the projection has at most 4 planes, so
 // no load goes out past them; 16 otherwise), the rest in a loop.
 template <int SP>
-__global__ __launch_bounds__(RW_THREADS) void k_resid_w(float* __restrict__ x, const float* __restrict__ part,
+__global__ __launch_bounds__(RW_THREADS) void k_resid_w(const float* x, float* xo, const float* __restrict__ part,
                                                       int splits, int M, int H, int round,
                                                       const float* __restrict__ w, int KU, uint4* __restrict__ Xp,
                                                       float* __restrict__ ssp) {
@@ -1219,7 +1292,7 @@ __global__ __launch_bounds__(RW_THREADS) void k_resid_w(float* __restrict__ x, c
             if (round)
                 xv = make_float4(round_f16_value(xv.x), round_f16_value(xv.y), round_f16_value(xv.z),
                                  round_f16_value(xv.w));
-            *(float4*)(x + xoff) = xv;
+            *(float4*)(xo + xoff) = xv;
         }
     }
     if (!w) return;   // the residual step alone (the pass's last block)
@@ -1247,15 +1320,159 @@ __global__ __launch_bounds__(RW_THREADS) void k_resid_w(float* __restrict__ x, c
     }
 }
 
-void launch_resid_w(hipStream_t st, float* x, const float* part, int splits, int M, int Mpad, int H, int round,
-                    const float* w, int KU, uint4* Xp, float* ssp) {
+void launch_resid_w(hipStream_t st, const float* x, float* xo, const float* part, int splits, int M, int Mpad, int H,
+                    int round, const float* w, int KU, uint4* Xp, float* ssp) {
     const int nsl = (H / 4 + RW_THREADS - 1) / RW_THREADS;
     const dim3 grid(nsl, w ? Mpad : M);
     if (splits <= 4)
-        hipLaunchKernelGGL(k_resid_w<4>, grid, dim3(RW_THREADS), 0, st, x, part, splits, M, H, round, w, KU, Xp, ssp);
+        hipLaunchKernelGGL(k_resid_w<4>, grid, dim3(RW_THREADS), 0, st, x, xo, part, splits, M, H, round, w, KU, Xp,
+                           ssp);
     else
-        hipLaunchKernelGGL(k_resid_w<RN_SPLITS>, grid, dim3(RW_THREADS), 0, st, x, part, splits, M, H, round, w, KU,
-                           Xp, ssp);
+        hipLaunchKernelGGL(k_resid_w<RN_SPLITS>, grid, dim3(RW_THREADS), 0, st, x, xo, part, splits, M, H, round, w,
+                           KU, Xp, ssp);
+    CHECK_LAUNCH();
+}
+
+// The residual step of k_resid_w on N columns of row m from column k0 (N and
+// k0 multiples of 4): x plus the planes in order, rounded on demand. Its
+// kernels pad the plane sum with +0 to 4 or 16 planes, which turns a sum of
+// -0 into +0: so does this one.
+template <int N>
+__device__ static inline void resid_row(const LxPro& p, int M, int H, int m, int k0, float (&x)[N]) {
+    const auto rp = __builtin_amdgcn_make_buffer_rsrc((void*)p.part, 0, p.splits * M * H * 4, 0x00020000);
+    const int at = (m * H + k0) * 4, plane = M * H * 4;
+    float s[N];
+#pragma unroll
+    for (int e = 0; e < N; e += 4) {
+        const float4 v = *(const float4*)(p.x + (size_t)m * H + k0 + e);
+        x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
+        s[e] = s[e + 1] = s[e + 2] = s[e + 3] = 0.0f;
+    }
+    for (int q = 0; q < p.splits; q += 4) {   // four planes' loads in flight; past the last one a load reads +0
+        u32x4 v[4][N / 4];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int e = 0; e < N / 4; e++) v[i][e] = __builtin_amdgcn_raw_buffer_load_b128(rp, at + 16 * e, (q + i) * plane, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int e = 0; e < N; e++) {
+                const float f = __uint_as_float(v[i][e / 4][e % 4]);
+                s[e] = q + i == 0 ? f : s[e] + f;
+            }
+    }
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+        if (p.splits > 4 && p.splits < 16) s[e] = s[e] + 0.0f;
+        x[e] = x[e] + s[e];
+        if (p.round) x[e] = round_f16_value(x[e]);
+    }
+}
+
+// The rest of k_resid_w for four (slice, row) pairs: the new rows to xo and
+// the slices' sums of squares. 128 threads a pair; red: 2 floats a pair.
+__device__ static void resid_slices(const LxPro& p, int M, int H, float* red) {
+    const int t = threadIdx.x % RW_THREADS, g = threadIdx.x / RW_THREADS, lane = t & 63;
+    const int nsl = (H / 4 + RW_THREADS - 1) / RW_THREADS;
+    const int i = (blockIdx.x - p.G) * 4 + g, m = i / nsl, sl = i % nsl;
+    const int c4 = sl * RW_THREADS + t;
+    const bool live = m < M && c4 < H / 4;
+    float x[4] = {0.f, 0.f, 0.f, 0.f};
+    if (live) {
+        resid_row<4>(p, M, H, m, 4 * c4, x);
+        *(float4*)(p.xo + (size_t)m * H + 4 * c4) = make_float4(x[0], x[1], x[2], x[3]);
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; e++) ss = ss + x[e] * x[e];
+    ss = wave_sum(ss);
+    if (lane == 0) red[2 * g + (t >> 6)] = ss;
+    __syncthreads();
+    if (t == 0 && m < M) p.ssp[(size_t)m * RW_SMAX + sl] = (0.0f + red[2 * g]) + red[2 * g + 1];
+}
+
+// k_fin_swiglu's 8 columns of row m from column k0, with the row factor f.
+__device__ static inline void swiglu8(const LxPro& p, int M, int m, int k0, float f, float (&v)[8]) {
+    const size_t N2 = 2 * (size_t)p.F, plane = (size_t)M * N2;
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = 0.0f;
+    if (k0 >= p.F) return;   // F is a multiple of 32: 8 columns are in or out together
+    float g[8], u[8];
+    const auto rp = __builtin_amdgcn_make_buffer_rsrc((void*)p.part, 0, (uint32_t)(p.splits * plane * 4), 0x00020000);
+    const int at = (int)(((size_t)m * N2 + k0) * 4);
+    for (int q = 0; q < p.splits; q += 4) {
+        u32x4 x[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int so = (int)((q + i) * plane * 4);
+            x[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rp, at, so, 0);
+            x[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rp, at + 16, so, 0);
+            x[i][2] = __builtin_amdgcn_raw_buffer_load_b128(rp, at + 4 * p.F, so, 0);
+            x[i][3] = __builtin_amdgcn_raw_buffer_load_b128(rp, at + 4 * p.F + 16, so, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (q + i < p.splits)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float a = __uint_as_float(x[i][e >> 2][e & 3]), b = __uint_as_float(x[i][2 + (e >> 2)][e & 3]);
+                    g[e] = q + i == 0 ? a : g[e] + a;
+                    u[e] = q + i == 0 ? b : u[e] + b;
+                }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        g[e] = g[e] * f;
+        u[e] = u[e] * f;
+        const float sc = 1.0f / (1.0f + expf(-g[e]));
+        v[e] = g[e] * sc * u[e];
+    }
+}
+
+// Whether w's matmul at M rows forms its operand itself: yes while what each
+// workgroup then reads, its columns of `values` f32 planes of M rows, is at
+// most this. Reading it is the cost: a launch saved is about 3 us, and a
+// workgroup's share comes in at about 100 KB/us once its 511 neighbours read
+// theirs from the L2s too. Passes measured with the line swept from 0 to 4 MB,
+// none fused against the best line against every one fused, us:
+//   hidden 576,  8 blocks:  1 row 384/313/313, 4: 388/325/326, 16: 414/375/375
+//   hidden 4096, 4 blocks:  1 row 368/334/334, 4: 384/364/365, 8: 401/395/401,
+//                           12: 417/415/436, 16: 433/433/469
+//   hidden 5120, 3 blocks:  1 row 348/319/319, 4: 360/348/349, 8: 379/375/381,
+//                           12: 395/395/417, 16: 411/411/449
+// The best line is 256 KB in every one of them, to within their noise of
+// 0.3%; at 384 KB and past it the passes of 8 to 16 rows lose.
+constexpr size_t LX_PRO_BYTES = 256 << 10;
+bool gemm_fuses(const QTensor& w, int M, int values) {
+    const int len = (w.KU + w.P - 1) / w.P;
+    return M <= GEMM_FUSE_ROWS && (size_t)M * values * len * 256 <= LX_PRO_BYTES;
+}
+
+void launch_gemm_resid(hipStream_t st, const QTensor& w, const float* x, float* xo, const float* part, int splits,
+                       int round, const float* norm, float* ssp, float* out, int M, int ncu) {
+    LxPro p;
+    p.part = part;
+    p.splits = splits;
+    p.x = x;
+    p.xo = xo;
+    p.w = norm;
+    p.round = round;
+    p.ssp = ssp;
+    if (w.f32s) launch_lx<1, true, LX_PRO_RESID>(st, w, nullptr, out, M, ncu, p);
+    else launch_lx<1, false, LX_PRO_RESID>(st, w, nullptr, out, M, ncu, p);
+    CHECK_LAUNCH();
+}
+
+void launch_gemm_swiglu(hipStream_t st, const QTensor& w, const float* part, int splits, int F, const RowScale& rs,
+                        float* out, int M, int ncu) {
+    LxPro p;
+    p.part = part;
+    p.splits = splits;
+    p.rs = rs;
+    p.F = F;
+    if (w.f32s) launch_lx<1, true, LX_PRO_SWIGLU>(st, w, nullptr, out, M, ncu, p);
+    else launch_lx<1, false, LX_PRO_SWIGLU>(st, w, nullptr, out, M, ncu, p);
     CHECK_LAUNCH();
 }
 

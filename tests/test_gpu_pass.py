@@ -236,6 +236,34 @@ def test_packed_by_many_workgroups_equals_alone(gpu, njobs, longest, nverify):
         c.close()
 
 
+@pytest.mark.parametrize("shape,blocks,rows", [("SMOLLM2", 3, (1, 2, 5, 15, 16)), ("LLAMA8B", 2, (1, 2, 3, 6, 8, 9, 16)),
+                                                ("M27B", 2, (1, 3, 4, 7, 12, 16)), ("QWEN38", 4, (1, 2, 4, 7, 16))])
+def test_few_rows_form_their_own_operands_to_the_same_bits(gpu, shape, blocks, rows):
+    """At few rows a matmul forms its operand itself from the planes before it
+    (the residual step, SwiGLU), by a rule on rows, planes and width: on both
+    sides of it, with one block (no carry from block to block) and with
+    several, a pass's rows are the bits they are in a pass of 17 rows, where
+    no matmul does."""
+    from chattorrent_amd.ccdecode import Context
+    rng = np.random.default_rng(blocks)
+    d = configs.with_layers(getattr(configs, shape), blocks)
+    c = Context(d, n_max=64, t_max=17, slots=5, lo=1, hi=1 + blocks)
+    try:
+        c.fill_random(SEED)
+        for n in rows:
+            cuts = [n] if n < 4 else [1, n - 3, 2]     # one chat, or decode rows beside a longer chunk
+            jobs = [dict(slot=s, past=0, n=k, hidden=rng.standard_normal((k, d["hidden"])).astype(np.float16)
+                         .view(np.uint16)) for s, k in enumerate(cuts)]
+            rest = dict(slot=4, past=0, n=17 - n, hidden=np.zeros((17 - n, d["hidden"]), np.uint16))
+            for to in (2, 1 + blocks):
+                got = c.step(jobs, at=1, to=to)
+                want = c.step(jobs + [rest], at=1, to=to)
+                for g, w in zip(got, want):
+                    assert np.array_equal(g, w), (n, to)
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("rows", [(1,), (127,), (128, 129), (300, 277)])
 def test_rows_in_and_out_in_pieces(gpu, rows):
     """f16 rows cross to and from the device in 1 MB pieces (128 rows of 4096
