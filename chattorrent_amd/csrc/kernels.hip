@@ -3079,10 +3079,221 @@ __global__ __launch_bounds__(256, NG > 4 ? 1 : 2) void k_attn(const AttnItem* __
     }
 }
 
+// Few items, each of one m-tile: a workgroup an item. Alone, a wave of
+// attn_item dequantises a page's 64 x D codes twice over (K and V) in about
+// 2.6 us, and a chat's chunks leave most of the GPU's SIMDs without one. Here
+// wave w takes the page's K token tile w and the V d-tiles w*DT/4 .., with
+// their scales straight into registers; the scores cross in LDS, one barrier
+// a page (two buffers: a wave past page p's barrier has read page p - 1's),
+// and every wave goes through the whole softmax. A page's share is a quarter
+// of the registers, so two pages are on their way. Bound by that chain: 9000
+// tokens of one chat (144 items of 8 pages, head_dim 128) 22.5 -> 14.5 us a
+// launch. Every value and every operation of a row is the one attn_item
+// computes for it.
+template <int NG>
+__global__ __launch_bounds__(256, 1) void k_attn_wide(const AttnItem* __restrict__ items, const uint4* __restrict__ Qp,
+                                                      const uint8_t* __restrict__ kpool,
+                                                      const uint8_t* __restrict__ vpool,
+                                                      const uint32_t* __restrict__ page_table, KVGeom g, int group,
+                                                      int ppw, float* __restrict__ part) {
+    constexpr int D = 32 * NG, DT = D / 16, DW = DT / 4, NB = NG > 4 ? NG / 4 : 1;   // d-tiles, 32-blocks a wave
+    __shared__ float4_t s_p[2][4][64];
+    __shared__ int s_big[2][4];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, j4 = lane >> 4, l16 = lane & 15;
+    const AttnItem it = items[blockIdx.x];
+    if (it.mt < 0) return;   // the whole workgroup
+    const int T_act = it.past + it.n;
+    const int R = it.n * group;
+    const int npg = (T_act + 63) >> 6;
+    const int p0 = it.p0, p1 = min(npg, p0 + ppw);
+    const float score_scale = 1.4426950408889634f / sqrtf((float)D);
+    const int b0 = wv * DW / 2;   // the wave's first 32-block of V
+    const uint32_t* pt = page_table + (size_t)it.slot * g.max_pages;
+    const uint32_t pgv = lane < p1 - p0 ? pt[p0 + lane] : 0u;
+    const size_t hoff = (size_t)it.kvh * g.blk, pstride = (size_t)g.nKV * g.blk;
+    // a page past the chunk's last: a resource of no bytes, whose loads read zero
+    auto page_rsrc = [&](const uint8_t* pool, int p) {
+        const uint32_t pg = __builtin_amdgcn_readlane(pgv, p < p1 ? p - p0 : 0);
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(pool + (size_t)pg * pstride + hoff), 0, p < p1 ? g.blk : 0,
+                                                 0x00020000);
+    };
+    const int vk = l16 * D + (D / 4) * j4, vv = j4 * D * 16 + l16 * 16;
+    struct Page {
+        u32x4 kc[NG / 2], ks[NG], vc[DW], vs[NB][4];
+    };
+    auto load_k = [&](Page& g1, int p) {
+        const auto rk = page_rsrc(kpool, p);
+#pragma unroll
+        for (int q = 0; q < NG / 2; q++)
+            g1.kc[q] = __builtin_amdgcn_raw_buffer_load_b128(rk, vk, wv * 16 * D + 16 * q, NG > 4 ? 0 : 2);
+        // tokens 16 wv + 4 j4 + r, groups 0..NG-1
+#pragma unroll
+        for (int q = 0; q < NG; q++)
+            g1.ks[q] = __builtin_amdgcn_raw_buffer_load_b128(rk, j4 * 16 * NG + 16 * q, 64 * D + wv * 64 * NG, 0);
+    };
+    auto load_v = [&](Page& g1, int p) {
+        const auto rv = page_rsrc(vpool, p);
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                g1.vs[b][q] = __builtin_amdgcn_raw_buffer_load_b128(rv, j4 * 64 * NG + 16 * q, 64 * D + (b0 + b) * 64, 0);
+#pragma unroll
+        for (int i = 0; i < DW; i++)
+            g1.vc[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, vv, (wv * DW + i) * 256, NG > 4 ? 0 : 2);
+    };
+    Page pa, pb;
+    load_k(pa, p0);
+    load_v(pa, p0);
+    load_k(pb, p0 + 1);
+    load_v(pb, p0 + 1);
+    uint4 qh[NG], ql[NG];
+#pragma unroll
+    for (int gg = 0; gg < NG; gg++) {
+        qh[gg] = Qp[(size_t)it.qb + lane + (size_t)gg * 128];
+        ql[gg] = Qp[(size_t)it.qb + lane + (size_t)gg * 128 + 64];
+    }
+    const int rho = it.mt * 16 + l16;
+    const int lim = rho < R ? it.past + rho / group : -1;
+    float mrow = -INFINITY, lsum = 0.0f;
+    bool shifted = true;
+    float4_t o[DW];
+#pragma unroll
+    for (int i = 0; i < DW; i++) o[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    auto page = [&](Page& g1, int p, int buf) {
+        // the scores of this wave's token tile
+        float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int gg = 0; gg < NG; gg++) {
+            const u32x4 c = g1.kc[gg >> 1];
+            const half8_t kf = (gg & 1) ? dequant8_biased(c[2], c[3]) : dequant8_biased(c[0], c[1]);
+            float4_t pp = {0.f, 0.f, 0.f, 0.f};
+            pp = mfma16x16x32(kf, __builtin_bit_cast(half8_t, qh[gg]), pp);
+            pp = mfma16x16x32(kf, __builtin_bit_cast(half8_t, ql[gg]), pp);
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                acc[r] = __builtin_fmaf(__uint_as_float(g1.ks[(r * NG + gg) >> 2][(r * NG + gg) & 3]), pp[r], acc[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[r] = acc[r] * score_scale;
+        if (p * 64 + 63 > it.past) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int tok = p * 64 + wv * 16 + 4 * j4 + r;
+                if (!(tok < T_act && tok <= lim)) acc[r] = -INFINITY;
+            }
+        }
+        s_p[buf][wv][lane] = acc;
+        load_k(g1, p + 2);
+        bool big = false;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (p * 64 + 64 > T_act) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (p * 64 + 16 * q + 4 * j4 + e >= T_act) g1.vs[b][q][e] = 0u;
+                }
+                big = big || pv_big(g1.vs[b][q]);
+            }
+        const bool wbig = __builtin_amdgcn_ballot_w64(big) != 0;
+        if (lane == 0) s_big[buf][wv] = wbig;
+        __syncthreads();
+        float pr[4][4];
+        float pm = -INFINITY;
+        bool pbig = false;
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++) {
+            const float4_t v = s_p[buf][tt][lane];
+            pbig = pbig || s_big[buf][tt] != 0;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                pr[tt][r] = v[r];
+                pm = fmaxf(pm, pr[tt][r]);
+            }
+        }
+        pm = fmaxf(pm, __shfl_xor(pm, 16));
+        pm = fmaxf(pm, __shfl_xor(pm, 32));
+        const float mnew = fmaxf(mrow, pm);
+        const bool drop = pbig || !(fabsf(mnew) < PV_MAX_SCORE);
+        const float shrink = drop && shifted ? PV_UNSHIFT : 1.0f;
+        shifted = shifted && !drop;
+        const float alpha = (mrow == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mrow - mnew)) * shrink;
+        lsum *= alpha;
+#pragma unroll
+        for (int i = 0; i < DW; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[i][r] *= alpha;
+        const float msub = (mnew == -INFINITY ? 0.0f : mnew) - (shifted ? PV_SHIFT_LOG2 : 0.0f);
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float e = __builtin_amdgcn_exp2f(pr[tt][r] - msub);
+                pr[tt][r] = e;
+                lsum += e;
+            }
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                u32x4 phw, plw;
+#pragma unroll
+                for (int ii = 0; ii < 8; ii += 2) {
+                    const int tt = 2 * ks + (ii >> 2), r = ii & 3;
+                    uint32_t h, l;
+                    split_hilo2(pr[tt][r] * __uint_as_float(g1.vs[b][tt][r]),
+                                pr[tt][r + 1] * __uint_as_float(g1.vs[b][tt][r + 1]), h, l);
+                    phw[ii >> 1] = h;
+                    plw[ii >> 1] = l;
+                }
+                const half8_t ph = __builtin_bit_cast(half8_t, phw), pl = __builtin_bit_cast(half8_t, plw);
+#pragma unroll
+                for (int i = b * DW / NB; i < (b + 1) * DW / NB; i++) {
+                    const u32x4 c = g1.vc[i];
+                    const half8_t vf = ks ? dequant8_biased(c[2], c[3]) : dequant8_biased(c[0], c[1]);
+                    o[i] = mfma16x16x32(vf, ph, o[i]);
+                    o[i] = mfma16x16x32(vf, pl, o[i]);
+                }
+            }
+        mrow = mnew;
+        load_v(g1, p + 2);
+    };
+    for (int p = p0; p < p1; p += 2) {
+        page(pa, p, 0);
+        if (p + 1 < p1) page(pb, p + 1, 1);
+    }
+    lsum += __shfl_xor(lsum, 16);
+    lsum += __shfl_xor(lsum, 32);
+    if (rho < R) {
+        const float un = shifted ? PV_UNSHIFT : 1.0f;
+        float* dst = part + it.part + (size_t)l16 * (D + 4);
+#pragma unroll
+        for (int i = 0; i < DW; i++) *(float4_t*)(dst + 4 + (wv * DW + i) * 16 + 4 * j4) = o[i] * un;
+        if (wv == 0 && j4 == 0) *(float2*)dst = make_float2(mrow, lsum * un);
+    }
+}
+
 void launch_attn(hipStream_t st, const AttnItem* items, int nitems, const uint4* Qp,
                  const uint8_t* kpool, const uint8_t* vpool, const uint32_t* page_table, const KVGeom& g, int group,
                  int ppw, float* part, int multi, AttnSched& sc) {
     if (nitems <= 0) return;
+    // A workgroup an item while all are resident at once with a SIMD to each
+    // wave (head_dim 256, 64) or with two waves a SIMD (128). An attention
+    // launch here against k_attn's, us: head_dim 256, 32-256 items -10 to -18,
+    // 288 +10; head_dim 128, 32-256 items -7 to -8, 288-512 -4 to -2, 576 +6;
+    // head_dim 64 (items of 2 pages) 36-240 items -0.4 to -1.7, 258-516 within
+    // 0.6 either way, 576 +2.
+    if (!multi && nitems <= (g.ng == 4 ? 2 : 1) * sc.ncu) {
+        const auto kern = g.ng == 8 ? k_attn_wide<8> : g.ng == 4 ? k_attn_wide<4> : k_attn_wide<2>;
+        hipLaunchKernelGGL(kern, dim3(nitems), dim3(256), 0, st, items, Qp, kpool, vpool, page_table, g, group, ppw,
+                           part);
+        CHECK_LAUNCH();
+        return;
+    }
     const int nblk = (nitems + 3) / 4;
     const int cap = sc.ncu * (g.ng == 8 ? 1 : 2);   // workgroups resident at once
     // blocks past the first round go out from the counter while they are few;

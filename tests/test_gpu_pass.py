@@ -236,6 +236,35 @@ def test_packed_by_many_workgroups_equals_alone(gpu, njobs, longest, nverify):
         c.close()
 
 
+@pytest.mark.parametrize("shape,blocks,rows", [("SMOLLM2", 1, 5), ("LLAMA8B", 1, 4), ("QWEN38", 4, 2)])
+@pytest.mark.parametrize("past", [1, 62, 63, 64, 127, 511, 1023, 2500])
+def test_attention_few_items_same_bits_as_many(gpu, shape, blocks, rows, past):
+    """With few work items attention gives each four waves, with many one: a
+    chat's rows (one, and the most that one m-tile holds) get the same bits
+    alone and beside chats long enough for the other kernel, over contexts at
+    the edges of pages and of work items."""
+    from chattorrent_amd.ccdecode import Context
+    d = configs.with_layers(getattr(configs, shape), blocks)
+    rng = np.random.default_rng(past)
+    n_max = 16448
+    c = Context(d, n_max=n_max, t_max=16, slots=6, lo=blocks, hi=blocks + 1)   # one attention block
+    try:
+        c.fill_random(SEED)
+        hid = [rng.standard_normal((rows, d["hidden"])).astype(np.float16).view(np.uint16) for _ in range(6)]
+        for n in (1, rows):
+            out = []
+            for chats in (1, 6):
+                ctx = [past] + [n_max - rows] * (chats - 1)
+                for s in range(chats):
+                    c.fill_random_kv(s, ctx[s], SEED, s + 1)
+                jobs = [dict(slot=s, past=ctx[s], n=n if s == 0 else 1, hidden=hid[s][:n if s == 0 else 1])
+                        for s in range(chats)]
+                out.append(c.step(jobs, at=blocks, to=blocks + 1)[0])
+            assert np.array_equal(out[0], out[1]), n
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("shape,blocks,rows", [("SMOLLM2", 3, (1, 2, 5, 15, 16)), ("LLAMA8B", 2, (1, 2, 3, 6, 8, 9, 16)),
                                                 ("M27B", 2, (1, 3, 4, 7, 12, 16)), ("QWEN38", 4, (1, 2, 4, 7, 16))])
 def test_few_rows_form_their_own_operands_to_the_same_bits(gpu, shape, blocks, rows):
