@@ -314,6 +314,7 @@ struct StepPlan {
     // item list k_attn takes (blocks of m-tiles padded to 4)
     int T = 0, S = 0, nitems = 0, ncwg = 0, nlaunch = 0;
     int multi = 0;   // a job of several Q m-tiles (attention's shared-page blocks)
+    int chunks = 0;  // the most chunks of a job
     std::vector<JobDev> jobs;
     std::vector<AttnItem> items;
     std::vector<int32_t> row_job, plan, head_rows, cwg;
@@ -1086,7 +1087,7 @@ static void plan_jobs(cc_ctx* ctx, const cc_job* jobs, int njobs, StepPlan& p, b
     const int ng = ctx->geom.ng;
     size_t qp = 0;
     int row = 0, items = 0, cwg = 0, S = 0, nlaunch = 0;
-    p.multi = 0;
+    p.multi = p.chunks = 0;
     for (int j = 0; j < njobs; j++) {
         JobDev& jd = p.jobs[j];
         jd.slot = jobs[j].slot;
@@ -1106,6 +1107,7 @@ static void plan_jobs(cc_ctx* ctx, const cc_job* jobs, int njobs, StepPlan& p, b
         nlaunch += ctx->geom.nKV * jd.nchunk * (jd.mtq > 1 ? 4 * ceil_div(jd.mtq, 4) : 1);
         cwg += ctx->geom.nKV * jd.mtq;
         if (jd.mtq > 1) p.multi = 1;
+        p.chunks = std::max(p.chunks, (int)jd.nchunk);
         if (head) S += jobs[j].sampled;
         row += jd.n;
     }
@@ -1205,7 +1207,7 @@ struct PassMeta {
     const AttnItem* items = nullptr;
     const int32_t* row_job = nullptr;
     const int32_t* cwg = nullptr;
-    int njobs = 0, nitems = 0, ncwg = 0, nlaunch = 0, multi = 0;
+    int njobs = 0, nitems = 0, ncwg = 0, nlaunch = 0, multi = 0, chunks = 0;
 };
 
 static RowScale row_scale_of(const cc_ctx* ctx) {
@@ -1236,8 +1238,13 @@ static void attn_mid(cc_ctx* ctx, Layer& L, float* part, int T, const PassMeta& 
                    L.kpool, L.vpool, ctx->page_table, ctx->qp, row_scale_of(ctx), 1, 1, ex);
     launch_attn(st, pm.items, pm.nlaunch, ctx->qp, L.kpool, L.vpool, ctx->page_table, ctx->geom, ctx->group,
                 ctx->ppw, ctx->apart, pm.multi, ctx->attn);
+    const float* gate = ctx->hybrid ? ctx->gbuf : nullptr;
+    if (gemm_fuses_attn(L.o, T, pm.chunks)) {
+        launch_gemm_attn(st, L.o, pm.jobs, pm.row_job, ctx->apart, ctx->geom, ctx->group, gate, part, T, ctx->ncu);
+        return;
+    }
     launch_attn_combine(st, pm.jobs, ctx->apart, ctx->geom, nH, ctx->group, L.o.KU, ctx->xp_o, nullptr, pm.cwg,
-                        pm.ncwg, ctx->hybrid ? ctx->gbuf : nullptr);
+                        pm.ncwg, gate);
     launch_gemm(st, L.o, ctx->xp_o, ctx->mt_alloc, part, T, ctx->ncu);
 }
 
@@ -1287,6 +1294,7 @@ static void run_blocks(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, int
     pm.nitems = p.nitems;
     pm.nlaunch = p.nlaunch;
     pm.multi = p.multi;
+    pm.chunks = p.chunks;
     pm.ncwg = p.ncwg;
     const RowScale rs = row_scale_of(ctx);
     const int KUH = ceil_div(H, 64);   // every block's first matmul reads K = hidden
@@ -1927,6 +1935,7 @@ cc_status cc_mtp_draft(cc_ctx* ctx, int32_t slot, int32_t row, int32_t token, in
         pm.nitems = plans[k].nitems;
         pm.nlaunch = plans[k].nlaunch;
         pm.multi = plans[k].multi;
+        pm.chunks = plans[k].chunks;
         pm.ncwg = plans[k].ncwg;
         mtp_input(ctx, ids + k, ctx->mtp_in, 1);
         full_attn_half(ctx, ctx->mtpL, ctx->mx, 1, mpad_of(1), pm);

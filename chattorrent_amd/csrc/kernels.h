@@ -216,6 +216,11 @@ void launch_gemm_resid(hipStream_t st, const QTensor& w, const float* x, float* 
                        int round, const float* norm, float* ssp, float* out, int M, int ncu);
 void launch_gemm_swiglu(hipStream_t st, const QTensor& w, const float* part, int splits, int F, const RowScale& rs,
                         float* out, int M, int ncu);
+// ... or from attention's chunk partials (launch_attn_combine's), for jobs of
+// at most `chunks` chunks.
+bool gemm_fuses_attn(const QTensor& w, int M, int chunks);
+void launch_gemm_attn(hipStream_t st, const QTensor& w, const JobDev* jobs, const int32_t* row_job, const float* part,
+                      const KVGeom& g, int group, const float* gate, float* out, int M, int ncu);
 void launch_resid_norm(hipStream_t st, float* x, const int32_t* rows, const float* part, int splits, int M,
                        int Mpad, int H, int round, const float* w, float eps, int KU, uint4* Xp, float* y);
 // The attention launches of one stream: the CU count and a pair of device

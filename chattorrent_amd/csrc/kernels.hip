@@ -82,13 +82,15 @@ __device__ static inline float rec_scale(uint32_t word, int h) {
 // another buffer: the others still read the old ones) and the sums of squares.
 // The operand's rows past M stay whatever LDS held: a row of the product
 // depends on its own row alone, and rows past M are not stored.
+// LX_PRO_ATTN does the same with k_attn_combine's launch (gemm_fuses_attn).
 // Few rows leave each launch bound by its own start, drain and first loads:
-// three of a block's ten go. One chat: hidden 576, 30 blocks and head
-// 1233 -> 1088 us; hidden 5120, 4 blocks 501 -> 474 us.
+// three of a block's ten go, or four. One chat: hidden 576, 30 blocks and
+// head 1233 -> 1088 us, with attention's merge 1054 -> 977; hidden 5120, 4
+// blocks 501 -> 474 us.
 __device__ static inline float row_scale(const RowScale& rs, int m);
-constexpr int LX_PRO_NONE = 0, LX_PRO_RESID = 1, LX_PRO_SWIGLU = 2;
+constexpr int LX_PRO_NONE = 0, LX_PRO_RESID = 1, LX_PRO_SWIGLU = 2, LX_PRO_ATTN = 3;
 struct LxPro {
-    const float* part = nullptr;   // the previous projection's planes
+    const float* part = nullptr;   // the previous projection's planes (ATTN: the chunk partials)
     int splits = 0;
     const float* x = nullptr;      // RESID: residual rows, the new ones, the norm's weights
     float* xo = nullptr;
@@ -98,6 +100,10 @@ struct LxPro {
     int G = 0;                     // the matmul's workgroups
     RowScale rs;                   // SWIGLU: the row factor
     int F = 0;
+    const JobDev* jobs = nullptr;  // ATTN: the rows' jobs, the output gate or null, head_dim, query heads a KV head
+    const int32_t* row_job = nullptr;
+    const float* gate = nullptr;
+    int D = 0, group = 0;
 };
 struct LxNoPro {};
 template <int PRO>
@@ -108,6 +114,7 @@ template <int N>
 __device__ static inline void resid_row(const LxPro& p, int M, int H, int m, int k0, float (&x)[N]);
 __device__ static inline void swiglu8(const LxPro& p, int M, int m, int k0, float f, float (&v)[8]);
 __device__ static void resid_slices(const LxPro& p, int M, int H, float* red);
+__device__ static inline void combine4(const LxPro& p, int K, int m, int unit, int lane, float (&v)[4]);
 
 template <int MT, bool F32S, int PRO = LX_PRO_NONE>
 __global__ __launch_bounds__(64 * LX_WAVES) void k_gemm_lx(const uint8_t* __restrict__ Wr,
@@ -158,7 +165,25 @@ __global__ __launch_bounds__(64 * LX_WAVES) void k_gemm_lx(const uint8_t* __rest
         for (int i = 0; i < PW; i++) load_w(w[i], s[i]);
     }
     // Activations of this plane into LDS: block (u, mt, q) of 1 KiB, q = 2h + hl.
-    if constexpr (PRO != LX_PRO_NONE) {
+    if constexpr (PRO == LX_PRO_ATTN) {
+        // a wave's 64 columns of a row at a time
+        for (int i = wave; i < M * len; i += WAVES) {
+            const int m = i / len, u = i % len;
+            float v[4];
+            combine4(pro, 64 * KU, m, ua + u, lane, v);
+            if (lane < 16) {
+                _Float16 h[4], l[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) split_hilo_x(v[e], h[e], l[e]);
+                // columns 4 lane ..: half-group lane / 8, k-block (lane % 8) / 2, half of its 16 bytes
+                uint2* at = (uint2*)(xs + (u * 4 + 2 * (lane >> 3)) * 64 + m + 16 * ((lane & 7) >> 1)) + (lane & 1);
+                at[0] = make_uint2(__builtin_bit_cast(uint32_t, half2_t{h[0], h[1]}),
+                                   __builtin_bit_cast(uint32_t, half2_t{h[2], h[3]}));
+                at[128] = make_uint2(__builtin_bit_cast(uint32_t, half2_t{l[0], l[1]}),
+                                     __builtin_bit_cast(uint32_t, half2_t{l[2], l[3]}));
+            }
+        }
+    } else if constexpr (PRO != LX_PRO_NONE) {
         // a thread's 8 columns of a row at a time
         const int per = 8 * len;
         for (int i = threadIdx.x; i < M * per; i += 64 * WAVES) {
@@ -3473,6 +3498,89 @@ void launch_attn_combine(hipStream_t st, const JobDev* jobs, const float* part, 
     else
         hipLaunchKernelGGL(k_attn_combine<64>, dim3(nwg), dim3(1024), 0, st, jobs, part, g, nH, group, KU, Xp, ctx_out,
                            wg_job, gate);
+    CHECK_LAUNCH();
+}
+
+// k_attn_combine's 64 columns of row m from 64 * unit, by one wave, for at
+// most 64 chunks: lane c forms chunk c's weight, lanes 16 q .. 16 q + 15 merge
+// quarter q's chunks, 4 columns each, and the first 16 add the quarters in
+// order. The result is in lanes 0 .. 15 (columns 4 lane ..). The same values
+// by the same operations as k_attn_combine's.
+__device__ static inline void combine4(const LxPro& p, int K, int m, int unit, int lane, float (&v)[4]) {
+    const int k0 = 64 * unit, h = k0 / p.D, kvh = h / p.group;
+    const JobDev jb = p.jobs[p.row_job[m]];
+    const int rho = (m - jb.row0) * p.group + h % p.group, W = p.D + 4, nc = jb.nchunk;
+    const size_t pstride = (size_t)16 * W;
+    const float* base = p.part + (size_t)(jb.item0 + (kvh * jb.mtq + (rho >> 4)) * nc) * pstride + (rho & 15) * W;
+    const int sub = lane >> 4;
+    const float* src = base + 4 + k0 % p.D + 4 * (lane & 15);
+    const int ca = (sub * nc) / COMBINE_SPLIT, c1 = ((sub + 1) * nc) / COMBINE_SPLIT;
+    const int most = (nc + COMBINE_SPLIT - 1) / COMBINE_SPLIT;   // chunks of the longest quarter
+    float4 x[8];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) x[u] = c0 + u < c1 ? *(const float4*)(src + (c0 + u) * pstride) : float4{0, 0, 0, 0};
+    };
+    load(ca);
+    const float2 ml = lane < nc ? *(const float2*)(base + lane * pstride) : make_float2(-INFINITY, 0.0f);
+    const float M = wave_max(ml.x);
+    const float w = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - M);
+    float lloc = 0.0f;
+    if (lane < nc) lloc += ml.y * w;
+    const float L = wave_sum(lloc);
+    float O[4] = {0, 0, 0, 0};
+    for (int c = 0; c < most; c += 8) {
+        if (c) load(ca + c);
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const float wc = __shfl(w, (ca + c + u) & 63);
+            if (ca + c + u < c1) {
+                O[0] += x[u].x * wc; O[1] += x[u].y * wc; O[2] += x[u].z * wc; O[3] += x[u].w * wc;
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float a1 = __shfl_down(O[e], 16), a2 = __shfl_down(O[e], 32), a3 = __shfl_down(O[e], 48);
+        v[e] = ((O[e] + a1) + a2) + a3;
+        v[e] = v[e] / L;
+    }
+    if (p.gate && lane < 16) {
+        const float4 g = *(const float4*)(p.gate + (size_t)m * K + k0 + 4 * lane);
+        const float gv[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float sg = 1.0f / (1.0f + expf(-gv[e]));
+            v[e] = sg * v[e];
+        }
+    }
+}
+
+// Whether w's matmul at M rows merges attention's chunks itself: a wave forms
+// 64 columns of a row at a time, each behind dependent loads (the row's job,
+// its partials, the weights), so the workgroup's columns times rows count,
+// over its 8 waves. Up to 2 rounds it beats the launch it saves. A block, us
+// (rounds in brackets): hidden 576, 1 row 2.9 less (1), 4 rows 2.1 less (1),
+// 6 rows 1.4 less (2), 8 rows 0.6 less (2), 9-12 rows 0.9 to 1.4 more (3);
+// hidden 4096, 1 row 1.7 less (2), 2 rows 3 more (4). A lane holds one
+// chunk's weight: at most 64.
+constexpr int LX_ATTN_COLUMNS = 2 * LX_WAVES;
+bool gemm_fuses_attn(const QTensor& w, int M, int chunks) {
+    const int len = (w.KU + w.P - 1) / w.P;
+    return chunks <= 64 && M <= GEMM_FUSE_ROWS && M * len <= LX_ATTN_COLUMNS;
+}
+
+void launch_gemm_attn(hipStream_t st, const QTensor& w, const JobDev* jobs, const int32_t* row_job, const float* part,
+                      const KVGeom& g, int group, const float* gate, float* out, int M, int ncu) {
+    LxPro p;
+    p.part = part;
+    p.jobs = jobs;
+    p.row_job = row_job;
+    p.gate = gate;
+    p.D = g.D;
+    p.group = group;
+    if (w.f32s) launch_lx<1, true, LX_PRO_ATTN>(st, w, nullptr, out, M, ncu, p);
+    else launch_lx<1, false, LX_PRO_ATTN>(st, w, nullptr, out, M, ncu, p);
     CHECK_LAUNCH();
 }
 

@@ -265,6 +265,33 @@ def test_attention_few_items_same_bits_as_many(gpu, shape, blocks, rows, past):
         c.close()
 
 
+@pytest.mark.parametrize("shape,blocks,page_run,rows", [("SMOLLM2", 1, 2, (1, 5, 6, 12)), ("LLAMA8B", 1, 8, (1,)),
+                                                         ("QWEN38", 4, 8, (1,))])
+@pytest.mark.parametrize("chunks", [1, 2, 3, 5, 33, 63, 64, 65])
+def test_o_proj_merges_few_rows_chunks_to_the_same_bits(gpu, shape, blocks, page_run, rows, chunks):
+    """At few rows o_proj's workgroups merge attention's chunks themselves (up
+    to 64 of them, one a lane): a chat's rows (of one m-tile and of two) get
+    the bits they get in a pass of 17 rows, which merges them in a launch of
+    its own, around the last lane's chunk."""
+    from chattorrent_amd.ccdecode import Context
+    d = configs.with_layers(getattr(configs, shape), blocks)
+    rng = np.random.default_rng(chunks)
+    past = 64 * page_run * chunks - max(rows) - 3
+    c = Context(d, n_max=past + 64, t_max=17, slots=2, lo=blocks, hi=blocks + 1)   # one attention block
+    try:
+        c.fill_random(SEED)
+        for s in range(2):
+            c.fill_random_kv(s, past, SEED, s + 1)
+        hid = rng.standard_normal((17, d["hidden"])).astype(np.float16).view(np.uint16)
+        for n in rows:
+            job = dict(slot=0, past=past, n=n, hidden=hid[:n])
+            rest = dict(slot=1, past=0, n=17 - n, hidden=hid[n:])
+            got, want = c.step([job], at=blocks, to=blocks + 1)[0], c.step([job, rest], at=blocks, to=blocks + 1)[0]
+            assert np.array_equal(got, want), n
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("shape,blocks,rows", [("SMOLLM2", 3, (1, 2, 5, 15, 16)), ("LLAMA8B", 2, (1, 2, 3, 6, 8, 9, 16)),
                                                 ("M27B", 2, (1, 3, 4, 7, 12, 16)), ("QWEN38", 4, (1, 2, 4, 7, 16))])
 def test_few_rows_form_their_own_operands_to_the_same_bits(gpu, shape, blocks, rows):
