@@ -177,7 +177,10 @@ typedef struct cc_job {
  * Outputs: when `to` is past the last block (the head), `top_vals`/`top_ids`
  * receive `topk` candidates per sampled row (sampled rows in job order, best
  * first, ties to the lower id); otherwise `hidden_out` receives every row as
- * f16 bits [T, hidden]. `status` (optional, njobs) is set per job. */
+ * f16 bits [T, hidden]. `status` (optional, njobs) is set per job. A pass
+ * that fails leaves the outputs alone; only if the device itself stops while
+ * a large pass's rows are leaving it (CC_EDEVICE) may hidden_out hold a part
+ * of them. */
 cc_status cc_step(cc_ctx* ctx, const cc_job* jobs, int32_t njobs, int32_t at, int32_t to,
                   int32_t topk, float* top_vals, uint32_t* top_ids, uint16_t* hidden_out,
                   int32_t* status);

@@ -1,0 +1,75 @@
+"""The library's host side on the CPU, its HIP runtime replaced by a stand-in
+(hip_stand_in.cc) whose kernels do nothing and are logged by name: a pass
+whose launch fails, and which kernels a pass takes. What the kernels compute
+is the GPU tests' matter."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+PRELUDE = """
+import ctypes as C, json, re, sys
+import numpy as np
+sys.path.insert(0, %r)
+from chattorrent_amd import ccdecode as cc, configs
+hip = C.CDLL(%r)
+hip.stand_in_reset.argtypes = [C.c_long]
+hip.stand_in_launches.restype = C.c_char_p
+
+def launched():
+    return hip.stand_in_launches().decode().split()
+
+def rows(n, d):
+    return np.zeros((n, d["hidden"]), np.uint16)
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    """host(code): runs it in a process whose HIP runtime is the stand-in and returns its `out`."""
+    so = str(tmp_path_factory.mktemp("hip") / "stand_in.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I",
+                    os.path.join(ROCM, "include"), os.path.join(HERE, "hip_stand_in.cc"), "-o", so], check=True)
+
+    def run(code):
+        r = subprocess.run([sys.executable, "-c", PRELUDE % (ROOT, so) + code + "\nprint(json.dumps(out))"], cwd=ROOT,
+                           env=dict(os.environ, LD_PRELOAD=so), stdout=subprocess.PIPE, stderr=subprocess.PIPE,
+                           text=True, timeout=300)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return json.loads(r.stdout.splitlines()[-1])
+
+    return run
+
+
+@pytest.mark.parametrize("n", [5, 300])
+def test_failed_launch_leaves_the_callers_rows(host, n):
+    """Whichever launch of a pass fails, the call says so and hidden_out is
+    untouched, also where the rows leave in pieces (300 rows of 4096); the
+    next pass succeeds and writes it."""
+    out = host(f"""
+n = {n}
+d = configs.with_layers(configs.LLAMA8B, 1)
+c = cc.Context(d, n_max=320, t_max=n, slots=1, lo=1, hi=2)
+job = cc.Job(slot=0, n=n)
+given = rows(n, d)
+job.hidden = given.ctypes.data_as(C.POINTER(C.c_uint16))
+hid = np.empty_like(given)
+out = []
+def step(fail):
+    hip.stand_in_reset(fail)
+    hid[:] = 0x1234
+    return c.lib.cc_step(c.h, C.byref(job), 1, 1, 2, 0, None, None, hid.ctypes.data, None)
+ok = step(-1) or step(-1)   # the first takes the job's pages
+total = len(launched())
+for k in sorted({{0, 1, total // 2, total - 2, total - 1}}):
+    out.append([step(k), bool((hid == 0x1234).all())])
+out = dict(failed=out, before=ok, after=step(-1), written=bool((hid == 0).all()), launches=total)
+""")
+    assert out["before"] == 0 and out["after"] == 0 and out["written"] and out["launches"] > 8
+    assert out["failed"] == [[8, True]] * 5   # CC_EDEVICE
