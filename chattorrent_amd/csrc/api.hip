@@ -1299,7 +1299,14 @@ static void run_blocks(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, int
     const RowScale rs = row_scale_of(ctx);
     const int KUH = ceil_div(H, 64);   // every block's first matmul reads K = hidden
     int longest = 0;                   // a long job takes the row-parallel conv
-    for (const JobDev& jd : p.jobs) longest = std::max(longest, (int)jd.n);
+    GdnRows walk;
+    for (const JobDev& jd : p.jobs) {
+        const int w = std::max(0, (int)jd.keep) + jd.n;
+        longest = std::max(longest, (int)jd.n);
+        walk.walked += w;
+        walk.longest = std::max(walk.longest, w);
+        walk.verifies += jd.snap != 0;
+    }
     auto planes = [&](const QTensor& w) { return gemm_planes(w, T, ctx->ncu); };
     // With few rows (gemm_fuses) a matmul adds the planes before it to the
     // residual rows itself, or forms SwiGLU itself, in place of a launch
@@ -1329,7 +1336,7 @@ static void run_blocks(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, int
             else
                 launch_lin_conv(st, pa, planes(L.lin), T, pm.njobs, pm.jobs, rs, L.conv, lg, L.state, ctx->lraw,
                                 ctx->lrep);
-            launch_gdn(st, ctx->lraw, ctx->lrep, pm.njobs, pm.jobs, L.gp, lg, L.state, ctx->lcore, longest);
+            launch_gdn(st, ctx->lraw, ctx->lrep, pm.njobs, pm.jobs, L.gp, lg, L.state, ctx->lcore, walk, ctx->ncu);
             launch_lin_norm(st, ctx->lcore, ctx->lraw, L.gnorm, d.rms_eps, T, lg, L.out.KU, ctx->xp_v);
             gemm(L.out, ctx->xp_v);
         } else {

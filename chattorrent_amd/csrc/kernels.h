@@ -148,9 +148,13 @@ constexpr int LIN_SEQ_ROWS = 16;   // longest job the one-thread-per-channel con
 void launch_lin_conv_rows(hipStream_t st, const float* part, int splits, int M, int njobs, const int32_t* row_job,
                           const JobDev* jobs, const RowScale& rs, const float* conv, const LinGeom& lg, float* state,
                           float* lraw, float* lrep, float* lring);
-// longest: the most rows a job of the pass has (it chooses the kernel).
+// What the recurrence's jobs walk, kept rows among them: all jobs' rows, the
+// longest job's, and how many jobs are verifies (it chooses the kernel).
+struct GdnRows {
+    int walked = 0, longest = 0, verifies = 0;
+};
 void launch_gdn(hipStream_t st, const float* lraw, const float* lrep, int njobs, const JobDev* jobs,
-                const float* gp, const LinGeom& lg, float* state, float* core, int longest);
+                const float* gp, const LinGeom& lg, float* state, float* core, const GdnRows& rows, int ncu);
 // RMSNormGated per (row, value head) with the gated_norm weight, times
 // silu(z), into the out_proj operand (K = valueDim).
 void launch_lin_norm(hipStream_t st, const float* core, const float* lraw, const float* gnorm, float eps,

@@ -2094,7 +2094,7 @@ void launch_lin_conv_rows(hipStream_t st, const float* part, int splits, int M, 
 // column with DK/8 rows of it each, in registers for the whole job. Two
 // kernels, the same operations on the same operands in the same order, so a
 // row's bits depend on neither its job's length nor its batch-mates:
-//   k_gdn_few  a pass whose jobs have few rows (GDN_FEW): bound by the state's
+//   k_gdn_few  jobs of few rows (gdn_takes_few): bound by the state's
 //              read and write, so few registers (many workgroups to hide the
 //              reads), whole 128-byte rows of state a load, the columns' sums
 //              through LDS with a barrier a token;
@@ -2107,12 +2107,8 @@ void launch_lin_conv_rows(hipStream_t st, const float* part, int splits, int M, 
 //              walk.
 // A single kernel that formed the dot products of q and k beside the state's
 // and read each token's inputs as it came to them took 1.49 us a row of a
-// long job: 512 rows 759 us a block (48 heads of 128 x 128), now 203. 16
-// sessions at 1, 2, 3, 4 and 8 rows (of 3.3 MB read and twice written with
-// a verify's snapshot) took 31.6, 35.9, 41.6, 46.2 and 69.4 us; k_gdn_few
-// takes 32.7, 36.1, 41.0 and 46.0, k_gdn 50.9 at 3 and 4 rows and 55.2 at 8:
-// the line between them.
-constexpr int GDN_TV = 32, GDN_T = 256, GDN_CH = 16, GDN_KG = 8, GDN_FEW = 4;
+// long job: 512 rows 759 us a block (48 heads of 128 x 128), now 203.
+constexpr int GDN_TV = 32, GDN_T = 256, GDN_CH = 16, GDN_KG = 8;
 static_assert(LIN_SPEC_ROWS < GDN_CH, "a rollback's kept rows and the row after them fall in one chunk");
 // Sum over the eight lanes 8i .. 8i+7, in all of them:
 // ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7)).
@@ -2398,24 +2394,49 @@ __global__ __launch_bounds__(GDN_T, 3) void k_gdn(const float* __restrict__ lraw
     put_state(S);
 }
 
+// Which kernel a launch takes, from the rows its jobs walk (a rollback's kept
+// rows among them), their sum over the jobs and the longest job's, and the
+// verifies, which write the state twice. With many workgroups a CU the work
+// decides: k_gdn_few takes about 0.95 us a job and 0.37 a verify less than
+// k_gdn and 0.28 us a row more (48 heads of 128 x 128), so the line is three
+// rows a job on average, and a fourth for a verify. With few the longest
+// job's chain does, 0.9 us a row longer in k_gdn_few, against a start of k_gdn
+// that grows with the workgroups.
+// Launches of 48 heads of 128 x 128, k_gdn_few / k_gdn, us (16, 4 and 1 jobs):
+//   1 row 22.7/33.5, 7.0/9.2, 4.9/5.6         2 rows 28.1/35.2, 9.1/10.3, 5.5/6.1
+//   3 rows (2 of them kept) 34.1/36.0, 11.3/10.6, 6.6/6.2
+//   4 rows 40.0/38.0, 12.6/11.2, 7.8/6.8      8 rows 63.4/43.0, 20.7/14.2, 12.7/7.9
+//   verifies of 4 rows 46.7/50.5, 13.9/13.9, 8.6/7.5, of 5 51.9/51.0, 16.0/14.4, 9.9/8.2
+//   1 row after 8 kept ones 68.8/42.1, 22.2/13.3, 13.2/7.8
+//   5 rows beside 15 (3) jobs of one 24.3/33.8 (11.3/10.7), 17 beside 15 30.4/35.7, 32 beside 15 47.1/36.2
+// Over 426 mixes of 1-16 jobs of 1-48 rows (this shape, 16 heads of it, 32
+// heads of 64 x 64) the rule's choice takes 0.2% more than the better kernel
+// on average and 17% (1.4 us) at worst; a line on the longest job's new rows
+// alone (4) took 8% more on average and up to 94%.
+static bool gdn_takes_few(int njobs, const GdnRows& r, const LinGeom& lg, int ncu) {
+    const long long groups = (long long)njobs * lg.nV * ((lg.Dv + GDN_TV - 1) / GDN_TV);
+    return r.walked <= 3 * njobs + r.verifies && r.longest <= std::max(2LL, 2 * groups / ncu - 5);
+}
+
 template <int DK>
 static void launch_gdn_dk(hipStream_t st, const float* lraw, const float* lrep, int njobs, const JobDev* jobs,
-                          const float* gp, const LinGeom& lg, float* state, float* core, int longest) {
+                          const float* gp, const LinGeom& lg, float* state, float* core, bool few) {
     const dim3 grid((lg.Dv + GDN_TV - 1) / GDN_TV, lg.nV, njobs), blk(GDN_T);
-    if (longest <= GDN_FEW)
+    if (few)
         hipLaunchKernelGGL(k_gdn_few<DK>, grid, blk, 0, st, lraw, lrep, jobs, gp, lg, state, core);
     else
         hipLaunchKernelGGL(k_gdn<DK>, grid, blk, 0, st, lraw, lrep, jobs, gp, lg, state, core);
 }
 
 void launch_gdn(hipStream_t st, const float* lraw, const float* lrep, int njobs, const JobDev* jobs, const float* gp,
-                const LinGeom& lg, float* state, float* core, int longest) {
+                const LinGeom& lg, float* state, float* core, const GdnRows& rows, int ncu) {
     if (njobs <= 0) return;
+    const bool few = gdn_takes_few(njobs, rows, lg, ncu);
     switch (lg.Dk) {
-        case 16: launch_gdn_dk<16>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, longest); break;
-        case 32: launch_gdn_dk<32>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, longest); break;
-        case 64: launch_gdn_dk<64>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, longest); break;
-        default: launch_gdn_dk<128>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, longest); break;
+        case 16: launch_gdn_dk<16>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, few); break;
+        case 32: launch_gdn_dk<32>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, few); break;
+        case 64: launch_gdn_dk<64>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, few); break;
+        default: launch_gdn_dk<128>(st, lraw, lrep, njobs, jobs, gp, lg, state, core, few); break;
     }
     CHECK_LAUNCH();
 }

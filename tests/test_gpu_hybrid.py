@@ -136,6 +136,37 @@ def test_hybrid_recurrence_same_bits_in_both_kernels(gpu, dk, dv):
         assert np.array_equal(g.view(np.uint32), got[0].view(np.uint32))
 
 
+@pytest.mark.parametrize("dk,dv", [(16, 16), (32, 48), (64, 32), (128, 64), (128, 128)])
+def test_hybrid_kept_rows_same_bits_in_both_kernels(gpu, dk, dv):
+    """A job after a rejected verify alone takes the long jobs' recurrence
+    kernel once it walks three rows (kept ones among them), and beside 39
+    one-row jobs the other one: the same bits, its own rows and the next row,
+    which reads the state it left."""
+    from chattorrent_amd.ccdecode import Context
+    d = dict(HW.SPIKE, n_layer=1, layer_types=["linear_attention"], lin_nk=16, lin_nv=48, lin_dk=dk, lin_dv=dv)
+    rng = np.random.default_rng(dv)
+    hid = rng.standard_normal((64, d["hidden"])).astype(np.float16).view(np.uint16)
+    c = Context(d, n_max=64, t_max=64, slots=40, sessions=40, lo=1, hi=2)
+    try:
+        c.fill_random(SEED)
+        past = 0
+        for keep, n in ((0, 1), (1, 1), (0, 3), (3, 1), (8, 1), (5, 4)):
+            out = []
+            for mates in (0, 39):
+                c.step([dict(slot=0, past=0, n=9, hidden=hid[:9])], at=1, to=2)
+                c.step([dict(slot=0, past=9, n=8, hidden=hid[9:17], snap=True)], at=1, to=2)
+                at = 9 + keep
+                got = c.step([dict(slot=0, past=at, n=n, hidden=hid[20:20 + n], keep=keep)] +
+                             [dict(slot=s, past=past, n=1, hidden=hid[s:s + 1]) for s in range(1, 1 + mates)],
+                             at=1, to=2)[:n]
+                past += mates > 0
+                out.append(np.concatenate([got, c.step([dict(slot=0, past=at + n, n=1, hidden=hid[30:31])], at=1,
+                                                       to=2)]))
+            assert np.array_equal(out[0], out[1]), (keep, n)
+    finally:
+        c.close()
+
+
 def test_hybrid_batch_mates_do_not_change_bits(gpu):
     """A session's logits do not depend on the other sessions packed with it."""
     d = HW.WIDE

@@ -73,3 +73,33 @@ out = dict(failed=out, before=ok, after=step(-1), written=bool((hid == 0).all())
 """)
     assert out["before"] == 0 and out["after"] == 0 and out["written"] and out["launches"] > 8
     assert out["failed"] == [[8, True]] * 5   # CC_EDEVICE
+
+
+@pytest.mark.parametrize("jobs,few", [
+    ([(0, 1)], True), ([(0, 2)], True), ([(0, 3)], False), ([(1, 1)], True), ([(2, 1)], False), ([(8, 1)], False),
+    ([(0, 2)] * 4, True), ([(0, 4)] * 4, False), ([(2, 1)] * 4, False),
+    ([(0, 3)] * 16, True), ([(0, 4)] * 16, False), ([(2, 1)] * 16, True), ([(3, 1)] * 16, False),
+    ([(0, 5)] + [(0, 1)] * 15, True), ([(0, 19)] + [(0, 1)] * 15, True), ([(0, 20)] + [(0, 1)] * 15, False),
+    ([(8, 1)] + [(0, 1)] * 15, True), ([(8, 1)] * 8 + [(0, 1)] * 8, False), ([("verify", 4)] * 16, True),
+    ([("verify", 5)] * 16, False), ([("verify", 4)] * 8 + [(0, 1)] * 8, True)])
+def test_recurrence_kernel_by_the_rows_walked(host, jobs, few):
+    """Each job is (kept rows, or a verify; new rows): a rollback's kept rows
+    are walked too, and a long job among many short ones does not move them
+    all to the long jobs' kernel. 48 heads of 128 x 128 on 256 CUs."""
+    out = host(f"""
+jobs = {jobs}
+d = dict(configs.QWEN38, n_layer=1, layer_types=["linear_attention"], mtp_vocab=0)
+c = cc.Context(d, n_max=64, t_max=256, slots=len(jobs), sessions=len(jobs), lo=1, hi=2)
+def step(**kw):
+    c.step([dict(slot=s, n=kw["n"][s], past=kw["past"][s], hidden=rows(kw["n"][s], d), snap=bool(kw["snap"][s]),
+                 keep=kw["keep"][s]) for s in range(len(jobs))], at=1, to=2)
+J, verify = len(jobs), [k == "verify" for k, _ in jobs]
+kept = [0 if v else k for v, (k, _) in zip(verify, jobs)]
+first = [8 if k else 1 for k in kept]
+step(n=[9] * J, past=[0] * J, snap=[0] * J, keep=[None] * J)
+step(n=first, past=[9] * J, snap=kept, keep=[None] * J)
+hip.stand_in_reset(-1)
+step(n=[n for _, n in jobs], past=[9 + (k or 1) for k in kept], snap=verify, keep=[k or None for k in kept])
+out = [k for k in launched() if "k_gdn" in k]
+""")
+    assert len(out) == 1 and ("k_gdn_few" in out[0]) == few, out
