@@ -1272,6 +1272,25 @@ static void ffn_half(cc_ctx* ctx, Layer& L, float* x, int T, int Mpad) {
 
 static int mpad_of(int T) { return 16 * ceil_div(T, 16) + (ceil_div(T, 16) > 1 && (ceil_div(T, 16) & 1) ? 16 : 0); }
 
+// Which of block b's matmuls form their operand themselves (gemm_fuses) in a
+// pass of T rows from block b0 on: the first one (from the block before's
+// planes), gate|up and down. run_blocks launches by it, and so does the
+// profile's replay.
+struct BlockFuse {
+    bool first, gu, down;
+};
+
+static BlockFuse block_fuse(const cc_ctx* ctx, int b, int b0, int T) {
+    const Layer& L = ctx->layers[b - ctx->L0];
+    const bool lin = L.kind == CC_LINEAR_ATTENTION;
+    auto planes = [&](const QTensor& w) { return gemm_planes(w, T, ctx->ncu); };
+    BlockFuse f;
+    f.first = b > b0 && gemm_fuses(lin ? L.lin : L.qkv, T, planes(ctx->layers[b - 1 - ctx->L0].down) + 1);
+    f.gu = gemm_fuses(L.gu, T, planes(lin ? L.out : L.o) + 1);
+    f.down = gemm_fuses(L.down, T, 2 * planes(L.gu));
+    return f;
+}
+
 // The blocks [p0, p1) (model indices) over the packed rows: blockSegs
 // (web/model/model.js:619-624) per layer, with the reference's dispatches
 // fused into: operand prep, q|k|v GEMM, finish (rmsnorm's row factor + RoPE +
@@ -1319,12 +1338,12 @@ static void run_blocks(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, int
         std::swap(x, x2);
         std::swap(pa, pb);
     };
-    bool pending = false;   // the last block's down planes wait for this block's first matmul
+    BlockFuse f = block_fuse(ctx, b0, b0, T);
     for (int b = b0; b < b1; b++) {
         Layer& L = ctx->layers[b - ctx->L0];
         const QTensor& w1 = L.kind == CC_LINEAR_ATTENTION ? L.lin : L.qkv;
         if (b == b0) launch_resid_w(st, x, x, nullptr, 0, T, Mpad, H, 0, L.ln1, KUH, ctx->xp_h, ctx->ssp);
-        if (pending) gemm_resid(w1, ctx->layers[b - 1 - ctx->L0].down, 1, L.ln1);
+        if (f.first) gemm_resid(w1, ctx->layers[b - 1 - ctx->L0].down, 1, L.ln1);
         else gemm(w1, ctx->xp_h);
         if (L.kind == CC_LINEAR_ATTENTION) {
             // linearBlockSegs (model.js:472-527): in_proj, conv + ring, the
@@ -1343,23 +1362,23 @@ static void run_blocks(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, int
             attn_mid(ctx, L, pa, T, pm);
         }
         const QTensor& w2 = L.kind == CC_LINEAR_ATTENTION ? L.out : L.o;
-        if (gemm_fuses(L.gu, T, planes(w2) + 1)) gemm_resid(L.gu, w2, 0, L.ln2);
+        if (f.gu) gemm_resid(L.gu, w2, 0, L.ln2);
         else {
             launch_resid_w(st, x, x, pa, planes(w2), T, Mpad, H, 0, L.ln2, KUH, ctx->xp_h, ctx->ssp);
             gemm(L.gu, ctx->xp_h);
         }
-        if (gemm_fuses(L.down, T, 2 * planes(L.gu))) {
+        if (f.down) {
             launch_gemm_swiglu(st, L.down, pa, planes(L.gu), d.ffn, rs, pb, T, ctx->ncu);
             std::swap(pa, pb);
         } else {
             launch_fin_swiglu(st, pa, planes(L.gu), T, Mpad, d.ffn, L.down.KU, ctx->xp_f, rs);
             gemm(L.down, ctx->xp_f);
         }
-        pending = false;
         if (b + 1 < b1) {
-            const Layer& Ln = ctx->layers[b + 1 - ctx->L0];
-            pending = gemm_fuses(Ln.kind == CC_LINEAR_ATTENTION ? Ln.lin : Ln.qkv, T, planes(L.down) + 1);
-            if (!pending) launch_resid_w(st, x, x, pa, planes(L.down), T, Mpad, H, 1, Ln.ln1, KUH, ctx->xp_h, ctx->ssp);
+            f = block_fuse(ctx, b + 1, b0, T);
+            if (!f.first)
+                launch_resid_w(st, x, x, pa, planes(L.down), T, Mpad, H, 1, ctx->layers[b + 1 - ctx->L0].ln1, KUH, ctx->xp_h,
+                               ctx->ssp);
         } else {
             launch_resid_w(st, x, ctx->x, pa, planes(L.down), T, Mpad, H, 1, nullptr, 0, nullptr, ctx->ssp);
         }
@@ -1415,46 +1434,73 @@ static void mtp_fill(cc_ctx* ctx, const MetaLayout& ml, int Tm, int njobs) {
 // back-to-back on one stream start as the previous one ends, so the pair's
 // interval over n launches is n kernel durations with no marker between them
 // (a marker next to every launch costs each a few microseconds of gap). The
-// replays write only scratch the step has consumed (matmul planes, attention
-// partials) or, for the head, the same logits again from the same operand.
+// replays write only scratch the step has consumed (matmul planes, the second
+// residual rows, sums of squares, attention partials) or, for the head, the
+// same logits again from the same operand. A matmul that formed its operand
+// itself (block_fuse, gemm_fuses_attn) does so again, from whatever planes the
+// step has left.
 static void prof_replay(cc_ctx* ctx, const StepPlan& p, const MetaLayout& ml, int b0, int b1, bool head) {
     const cc_dims& d = ctx->d;
     hipStream_t st = ctx->stream;
     const int T = p.T;
     const JobDev* djobs = (const JobDev*)(ctx->d_meta + ml.jobs);
     const AttnItem* ditems = (const AttnItem*)(ctx->d_meta + ml.items);
+    const int32_t* drow_job = (const int32_t*)(ctx->d_meta + ml.row_job);
+    const RowScale rs = row_scale_of(ctx);
+    auto layer = [&](int b) -> Layer& { return ctx->layers[b - ctx->L0]; };
+    auto planes = [&](const QTensor& w) { return gemm_planes(w, T, ctx->ncu); };
+    auto gemm = [&](const QTensor& w, const uint4* xp) {
+        launch_gemm(st, w, xp, ctx->mt_alloc, ctx->part, T, ctx->ncu);
+    };
+    auto gemm_resid = [&](const QTensor& w, const QTensor& before, int round, const float* norm) {
+        launch_gemm_resid(st, w, ctx->x, ctx->x2, ctx->part, planes(before), round, norm, ctx->ssp, ctx->part2, T,
+                          ctx->ncu);
+    };
     // (a linear_attention block has no q|k|v, o or KV: its matmuls are not replayed)
-    auto blocks = [&](int kind, QTensor Layer::*w, const uint4* xp) {
+    auto blocks = [&](int kind, QTensor Layer::*w, auto&& one) {
         double bytes = 0;
         int n = 0;
         for (int b = b0; b < b1; b++)
-            if ((ctx->layers[b - ctx->L0].*w).codes) {
-                bytes += qbytes(ctx->layers[b - ctx->L0].*w);
+            if ((layer(b).*w).codes) {
+                bytes += qbytes(layer(b).*w);
                 n++;
             }
         if (n == 0) return;
         prof_mark(ctx, kind, n, bytes, [&] {
             for (int b = b0; b < b1; b++)
-                if ((ctx->layers[b - ctx->L0].*w).codes)
-                    launch_gemm(st, ctx->layers[b - ctx->L0].*w, xp, ctx->mt_alloc, ctx->part, T, ctx->ncu);
+                if ((layer(b).*w).codes) one(b, layer(b), block_fuse(ctx, b, b0, T));
         });
     };
     if (b1 > b0) {
-        blocks(CC_K_QKV, &Layer::qkv, ctx->xp_h);
+        blocks(CC_K_QKV, &Layer::qkv, [&](int b, Layer& L, const BlockFuse& f) {
+            if (f.first) gemm_resid(L.qkv, layer(b - 1).down, 1, L.ln1);
+            else gemm(L.qkv, ctx->xp_h);
+        });
         int nfull = 0;
-        for (int b = b0; b < b1; b++) nfull += ctx->layers[b - ctx->L0].kpool != nullptr;
+        for (int b = b0; b < b1; b++) nfull += layer(b).kpool != nullptr;
         if (p.nitems > 0 && nfull > 0)
             prof_mark(ctx, CC_K_ATTN, nfull, p.kv_bytes * nfull, [&] {
                 for (int b = b0; b < b1; b++) {
-                    const Layer& L = ctx->layers[b - ctx->L0];
+                    const Layer& L = layer(b);
                     if (!L.kpool) continue;
                     launch_attn(st, ditems, p.nlaunch, ctx->qp, L.kpool, L.vpool, ctx->page_table, ctx->geom,
                                 ctx->group, ctx->ppw, ctx->apart, p.multi, ctx->attn);
                 }
             });
-        blocks(CC_K_O, &Layer::o, ctx->xp_o);
-        blocks(CC_K_GU, &Layer::gu, ctx->xp_h);
-        blocks(CC_K_DOWN, &Layer::down, ctx->xp_f);
+        blocks(CC_K_O, &Layer::o, [&](int, Layer& L, const BlockFuse&) {
+            if (gemm_fuses_attn(L.o, T, p.chunks))
+                launch_gemm_attn(st, L.o, djobs, drow_job, ctx->apart, ctx->geom, ctx->group,
+                                 ctx->hybrid ? ctx->gbuf : nullptr, ctx->part, T, ctx->ncu);
+            else gemm(L.o, ctx->xp_o);
+        });
+        blocks(CC_K_GU, &Layer::gu, [&](int, Layer& L, const BlockFuse& f) {
+            if (f.gu) gemm_resid(L.gu, L.kind == CC_LINEAR_ATTENTION ? L.out : L.o, 0, L.ln2);
+            else gemm(L.gu, ctx->xp_h);
+        });
+        blocks(CC_K_DOWN, &Layer::down, [&](int, Layer& L, const BlockFuse& f) {
+            if (f.down) launch_gemm_swiglu(st, L.down, ctx->part, planes(L.gu), d.ffn, rs, ctx->part2, T, ctx->ncu);
+            else gemm(L.down, ctx->xp_f);
+        });
     }
     if (head) {
         const QTensor& hw = d.tied ? ctx->wte : ctx->lm_head;

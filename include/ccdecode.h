@@ -257,7 +257,9 @@ cc_status cc_stats_get(const cc_ctx* ctx, cc_stats* out);
  * pair (so no marker sits between launches); cc_profile_read returns the
  * summed milliseconds, the launch count and the algorithmic HBM bytes of
  * those launches (q8 weights at 1.0625 B per weight; KV rows at
- * D + 4*D/32 B). The step's results are unchanged. Enabling resets the sums. */
+ * D + 4*D/32 B). The launches are the step's own kernels: with few rows a
+ * matmul's time includes forming its operand where it did so itself. The
+ * step's results are unchanged. Enabling resets the sums. */
 enum { CC_K_QKV = 0, CC_K_O = 1, CC_K_GU = 2, CC_K_DOWN = 3, CC_K_HEAD = 4, CC_K_ATTN = 5, CC_K_COUNT = 6 };
 cc_status cc_profile(cc_ctx* ctx, int32_t enable);
 cc_status cc_profile_read(const cc_ctx* ctx, int32_t kind, double* ms, int64_t* launches, double* bytes);

@@ -103,3 +103,36 @@ step(n=[n for _, n in jobs], past=[9 + (k or 1) for k in kept], snap=verify, kee
 out = [k for k in launched() if "k_gdn" in k]
 """)
     assert len(out) == 1 and ("k_gdn_few" in out[0]) == few, out
+
+
+@pytest.mark.parametrize("shape,blocks,chats,rows,past", [
+    ("SMOLLM2", 3, 1, 1, 300), ("SMOLLM2", 3, 1, 1, 9000), ("SMOLLM2", 3, 4, 1, 100), ("SMOLLM2", 3, 1, 9, 100),
+    ("SMOLLM2", 2, 17, 1, 100), ("LLAMA8B", 2, 1, 1, 100), ("LLAMA8B", 2, 2, 3, 100), ("M27B", 2, 1, 1, 100),
+    ("M27B", 2, 4, 1, 100), ("M27B", 2, 1, 16, 100), ("M27B", 2, 40, 1, 100), ("QWEN38", 4, 1, 1, 0),
+    ("QWEN38", 4, 2, 8, 0)])
+def test_profile_replays_the_passs_own_matmuls(host, shape, blocks, chats, rows, past):
+    """cc_profile times the kernels that the pass ran: each class's launches
+    are the pass's, block by block, also where few rows let a matmul form its
+    operand itself. (A linear_attention block's first matmul and out_proj are
+    in no class.)"""
+    out = host(f"""
+chats, n, past = {chats}, {rows}, {past}
+d = configs.with_layers(configs.{shape}, {blocks})
+d["mtp_vocab"] = 0
+kinds = d.get("layer_types") or ["full_attention"] * {blocks}
+c = cc.Context(d, n_max=64 * (past // 64 + 2), t_max=chats * n, slots=chats, sessions=chats, lo=1, hi=1 + {blocks})
+jobs = [dict(slot=s, past=past, n=n, hidden=rows(n, d)) for s in range(chats)]
+def matmuls():
+    hip.stand_in_reset(-1)
+    c.step(jobs, at=1, to=1 + {blocks})
+    return [k for k in launched() if "k_gemm" in k]
+own = matmuls()
+c.profile(True)
+both = matmuls()
+out = dict(own=own, both=both, full=[k == "full_attention" for k in kinds])
+""")
+    own, full = out["own"], out["full"]
+    assert out["both"][:len(own)] == own and len(own) == 4 * blocks
+    block = [own[4 * b:4 * b + 4] for b in range(blocks)]
+    want = [block[b][i] for i in range(4) for b in range(blocks) if full[b] or i > 1]
+    assert out["both"][len(own):] == want
