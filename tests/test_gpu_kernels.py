@@ -301,8 +301,8 @@ def test_attend_vs_oracle(gpu):
 def test_attend_verify_rows_equal_one_row_bitwise(gpu, shape):
     """A verify job's rows (several Q m-tiles: the workgroup's four waves share
     each page's dequantised fragments) give the bits of the same rows attended
-    one at a time (one m-tile: each wave dequantises for itself), across a
-    page and chunk boundary (positions 505..512)."""
+    one at a time (one m-tile and few items: four waves share an item), across
+    a page and chunk boundary (positions 505..512)."""
     base = configs.M27B if shape == "27b" else D256
     d = configs.with_layers(base, 1)
     c = _ctx(gpu, d, n_max=1024, t_max=64, slots=2)
@@ -453,3 +453,76 @@ def test_attend_beyond_the_shifted_split(gpu):
                 assert np.array_equal(one.view(np.uint32), got[i:i + 1].view(np.uint32)), (base["hidden"], "hot", i)
         finally:
             c.close()
+
+
+# contexts whose one-m-tile rows make more work items (of 2 pages where K/V
+# rows are narrow, else 8) than the few-item kernel takes: one wave an item
+MANY_ITEMS = {"smollm2": (configs.SMOLLM2, 11050), "27b": (configs.M27B, 33420), "d256": (D256, 34000)}
+
+
+@pytest.mark.parametrize("shape", sorted(MANY_ITEMS))
+def test_attend_many_items(gpu, shape):
+    """Decode rows through the kernel that long contexts and full batches
+    take, one wave a work item: V scales of 300-5000 inside items, at their
+    edges and on the last, partly filled page (the dropped shift), queries
+    times 5000 (scores past 4096 in log2 units, the other bound of the shift),
+    and NaN, infinity and the largest values in the pool rows past the
+    context. Against the oracle within 2e-5 of max |out| (1e-2 at the hot
+    scores, as for few items); the poisoned rows change no bit; a verify's
+    rows through the shared-page blocks have the bits of the same rows alone."""
+    from oracle import lib as L
+    from oracle import model as Mo
+    base, tokens = MANY_ITEMS[shape]
+    d = configs.with_layers(base, 1)
+    D, nH, nKV = d["head_dim"], d["n_heads"], d["n_kv_heads"]
+    group, nv, pages = nH // nKV, 8, -(-(tokens + 8) // 64) + 1
+    assert nKV * (tokens // 64 // (2 if nKV * D <= 512 else 8)) > (512 if D == 128 else 256)
+    assert (tokens + nv) % 64, "stale rows in the last page"
+    end = 64 * pages
+    c = _ctx(gpu, d, n_max=end, t_max=64, slots=1)
+    try:
+        om = Mo.Model(d, n_slots=1, max_pages=pages)
+        c.fill_random_kv(0, end, 11, 3)
+        om.fill_random_kv(0, end, 11, 3)
+        pg = om.frames[0]["pages"]
+        big = {100: 300.0, 101: 5000.0, 511: 1000.0, 512: 700.0, tokens // 2: 2000.0, tokens - 1: 400.0}
+        bad = np.empty((end - tokens - nv, D // 4 + D // 32), np.uint32)
+        bad[:, :D // 4] = 0x7f7f7f7f                    # codes at their largest
+        bad[:, D // 4:] = np.array([0x7fc00000, 0x7f800000, 0xff800000, 0x7f7fffff] * D, np.uint32)[:D // 32]
+        for h in range(nKV):
+            for t, sc in big.items():
+                row = om.kv_rows(0, 1, 0, t, t + 1, h)
+                row[0, D // 4:].view(np.float32)[h % (D // 32)] = np.float32(sc)
+                c.write_kv(0, 1, 0, h, t, row)
+                at = ((int(pg[t // 64]) * nKV + h) * 64 + t % 64) * om.rw
+                om.V[0][at:at + om.rw] = row[0]
+
+        def want(q, past):
+            n = q.shape[0]
+            Qh = q.reshape(n, nH, D).transpose(1, 0, 2).copy()   # rope works in place
+            L.rope(Qh, D, past, om.tbl)
+            s = L.qk_scores(Qh, om.K[0], n, past + n, 64, D, nH, group, pg)
+            top = np.abs(s).max() * 1.4426950408889634
+            return L.attn_av(L.causal_softmax(s, past), om.V[0], D, 64, group, pg).transpose(1, 0, 2).reshape(n, -1), top
+
+        rng = np.random.default_rng(tokens)
+        q = rng.standard_normal((nv, nH * D)).astype(np.float32)
+        q[[2, 5]] *= 5000.0
+        one = [c.op_attend(0, 0, q[i:i + 1], tokens + i) for i in range(nv)]
+        for i in (0, 2, nv - 1):
+            w, top = want(q[i:i + 1], tokens + i)
+            assert (top > 2 * 4096) == (i == 2), "scores short of the bound"
+            err = np.abs(one[i] - w).max()
+            assert err <= (1e-2 if i == 2 else 2e-5) * max(1.0, np.abs(w).max()), (i, err)
+        many = c.op_attend(0, 0, q, tokens)
+        for which in (0, 1):
+            for h in range(nKV):
+                c.write_kv(0, which, 0, h, tokens + nv, bad)
+        assert np.array_equal(c.op_attend(0, 0, q, tokens).view(np.uint32), many.view(np.uint32))
+        for i in range(nv):
+            assert np.isfinite(one[i]).all()
+            assert np.array_equal(one[i].view(np.uint32), many[i:i + 1].view(np.uint32)), i
+        last = c.op_attend(0, 0, q[-1:], tokens + nv - 1)   # the poisoned rows follow its token
+        assert np.array_equal(last.view(np.uint32), one[-1].view(np.uint32))
+    finally:
+        c.close()

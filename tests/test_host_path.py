@@ -136,3 +136,26 @@ out = dict(own=own, both=both, full=[k == "full_attention" for k in kinds])
     block = [own[4 * b:4 * b + 4] for b in range(blocks)]
     want = [block[b][i] for i in range(4) for b in range(blocks) if full[b] or i > 1]
     assert out["both"][len(own):] == want
+
+
+@pytest.mark.parametrize("shape,tokens,wide", [
+    ("smollm2", 130, True), ("27b", 700, True), ("d256", 700, True),
+    ("smollm2", 11050, False), ("27b", 33420, False), ("d256", 34000, False)])
+def test_attention_kernel_by_the_items(host, shape, tokens, wide):
+    """Which kernel the attention tests of test_gpu_kernels.py reach with one
+    decode row: four waves an item while items are few, one wave an item at
+    the contexts of its many-item test."""
+    out = host(f"""
+sys.path.insert(0, {HERE!r})
+import test_gpu_kernels as K
+base, long = K.MANY_ITEMS[{shape!r}]
+tokens = {tokens}
+assert tokens < 1024 or tokens == long
+d = configs.with_layers(base, 1)
+c = cc.Context(d, n_max=64 * (tokens // 64 + 2), t_max=64, slots=1)
+c.fill_random_kv(0, tokens + 1, 1, 1)
+hip.stand_in_reset(-1)
+c.op_attend(0, 0, np.zeros((1, d["n_heads"] * d["head_dim"]), np.float32), tokens)
+out = [k for k in launched() if "k_attn" in k and "combine" not in k]
+""")
+    assert len(out) == 1 and ("k_attn_wide" in out[0]) == wide, out
