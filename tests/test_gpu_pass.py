@@ -265,16 +265,29 @@ def test_attention_few_items_same_bits_as_many(gpu, shape, blocks, rows, past):
         c.close()
 
 
-@pytest.mark.parametrize("shape,blocks,page_run,rows", [("SMOLLM2", 1, 2, (1, 5, 6, 12)), ("LLAMA8B", 1, 8, (1,)),
-                                                         ("QWEN38", 4, 8, (1,))])
+# the position of a full-attention block, its pages a work item, row counts
+MERGE_CASES = {"SMOLLM2": (1, 2, (1, 5, 6, 12)), "LLAMA8B": (1, 8, (1,)), "QWEN38": (4, 8, (1,)),
+               "WIDE": (2, 2, (1, 5, 8)), "D256": (4, 2, (1, 3, 9, 16))}
+
+
+def merge_dims(shape):
+    import hybrid_weights as HW
+    return dict(getattr(HW, shape)) if hasattr(HW, shape) else configs.with_layers(getattr(configs, shape),
+                                                                                   MERGE_CASES[shape][0])
+
+
+@pytest.mark.parametrize("shape", sorted(MERGE_CASES))
 @pytest.mark.parametrize("chunks", [1, 2, 3, 5, 33, 63, 64, 65])
-def test_o_proj_merges_few_rows_chunks_to_the_same_bits(gpu, shape, blocks, page_run, rows, chunks):
+def test_o_proj_merges_few_rows_chunks_to_the_same_bits(gpu, shape, chunks):
     """At few rows o_proj's workgroups merge attention's chunks themselves (up
     to 64 of them, one a lane): a chat's rows (of one m-tile and of two) get
     the bits they get in a pass of 17 rows, which merges them in a launch of
-    its own, around the last lane's chunk."""
+    its own, around the last lane's chunk. WIDE and D256 do it with the output
+    gate and heads of 128 and 256; QWEN38's o_proj is too wide to (which of
+    the cases do is test_host_path.py's matter)."""
+    blocks, page_run, rows = MERGE_CASES[shape]
     from chattorrent_amd.ccdecode import Context
-    d = configs.with_layers(getattr(configs, shape), blocks)
+    d = merge_dims(shape)
     rng = np.random.default_rng(chunks)
     past = 64 * page_run * chunks - max(rows) - 3
     c = Context(d, n_max=past + 64, t_max=17, slots=2, lo=blocks, hi=blocks + 1)   # one attention block

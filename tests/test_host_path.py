@@ -159,3 +159,31 @@ c.op_attend(0, 0, np.zeros((1, d["n_heads"] * d["head_dim"]), np.float32), token
 out = [k for k in launched() if "k_attn" in k and "combine" not in k]
 """)
     assert len(out) == 1 and ("k_attn_wide" in out[0]) == wide, out
+
+
+@pytest.mark.parametrize("shape", ["SMOLLM2", "LLAMA8B", "QWEN38", "WIDE", "D256"])
+def test_few_rows_merge_chunks_in_o_proj(host, shape):
+    """Which cases of test_gpu_pass.py's chunk-merging test take the merge
+    inside o_proj's matmul: up to 64 chunks, while a workgroup's columns times
+    rows are at most 16."""
+    out = host(f"""
+sys.path.insert(0, {HERE!r})
+import test_gpu_pass as P
+at, run, rws = P.MERGE_CASES[{shape!r}]
+d, out = P.merge_dims({shape!r}), []
+for chunks in (1, 64, 65):
+    past = 64 * run * chunks - max(rws) - 3
+    c = cc.Context(d, n_max=past + 64, t_max=17, slots=2, lo=at, hi=at + 1)
+    c.fill_random_kv(0, past, 1, 1)
+    for n in rws:
+        hip.stand_in_reset(-1)
+        c.step([dict(slot=0, past=past, n=n, hidden=rows(n, d))], at=at, to=at + 1)
+        k = launched()
+        inside = any(re.search("k_gemm_lxILi1ELb.ELi3E", x) for x in k)
+        assert inside != any("k_attn_combine" in x for x in k)
+        out.append([chunks, n, inside])
+""")
+    most = {"SMOLLM2": 8, "LLAMA8B": 1, "QWEN38": 0, "WIDE": 8, "D256": 16}[shape]
+    for chunks, n, inside in out:
+        assert inside == (chunks <= 64 and n <= most), (chunks, n)
+    assert any(i for _, _, i in out) == (most > 0)
