@@ -108,8 +108,9 @@ def test_hybrid_recurrence_same_bits_in_both_kernels(gpu, dk, dv):
     """Passes of few rows a job and longer jobs take different recurrence
     kernels: 45 rows of a prompt fed in any cuts (below, at and above the
     rule's line and the 16-row chunk, value columns ending inside a tile) give
-    the last row's logits bit for bit, and so does a verify rolled back by a
-    job on either side of the line."""
+    the last row's logits bit for bit, and so does a verify on either side of
+    the line (two rows walked, for one session) rolled back by a job on
+    either side."""
     d = dict(HW.SPIKE, lin_dk=dk, lin_dv=dv)
     rng = np.random.default_rng(dk)
     prompt = _ids(rng, 45, d["vocab"])
@@ -119,14 +120,15 @@ def test_hybrid_recurrence_same_bits_in_both_kernels(gpu, dk, dv):
             c.step([dict(slot=0, past=past, n=n, ids=prompt[past:past + n], sampled=1, **kw)], topk=2)
             return past + n
         got = []
-        for cuts in ([45], [1] * 45, [4] * 11 + [1], [5] * 9, [15, 1, 16, 13], [17, 28], [33, 8, 4]):
+        for cuts in ([45], [1] * 45, [2] * 22 + [1], [4] * 11 + [1], [5] * 9, [15, 1, 16, 13], [17, 28], [33, 8, 4]):
             past = 0
             for n in cuts:
                 past = feed(past, n)
             got.append(c.read_logits(1).copy())
-        for keep, after in ((0, 4), (3, 1), (3, 9), (8, 2), (8, 14)):
+        for rows, keep, after in ((8, 0, 4), (8, 3, 1), (8, 3, 9), (8, 8, 2), (8, 8, 14), (8, 1, 1), (8, 0, 2),
+                                  (2, 0, 2), (2, 1, 1), (2, 2, 1), (1, 0, 1)):
             past = feed(0, 20)
-            c.step([dict(slot=0, past=20, n=8, ids=prompt[20 + np.arange(8)], sampled=8, snap=True)], topk=2)
+            c.step([dict(slot=0, past=20, n=rows, ids=prompt[20 + np.arange(rows)], sampled=rows, snap=True)], topk=2)
             past = feed(20 + keep, after, keep=keep)
             feed(past, 45 - past)
             got.append(c.read_logits(1).copy())
