@@ -1194,13 +1194,6 @@ static cc_status grow(cc_ctx* ctx, const StepPlan& p) {
     return CC_OK;
 }
 
-// The blocks [p0, p1) (model indices) over the packed rows: blockSegs
-// (web/model/model.js:619-624) per layer, with the reference's dispatches
-// fused into: operand prep, q|k|v GEMM, finish (rmsnorm's row factor + RoPE +
-// KV store + Q operand), attention, combine (o_proj operand), o GEMM,
-// residual (+ operand x*ln2 and the row's sum of squares), gate|up GEMM,
-// finish (row factor + SwiGLU), down GEMM, residual (+ round_f16 + the next
-// block's operand x*ln1 and sum of squares).
 // Device pointers of a pass's metadata, and its counts.
 struct PassMeta {
     const JobDev* jobs = nullptr;

@@ -85,8 +85,8 @@ __device__ static inline float rec_scale(uint32_t word, int h) {
 // LX_PRO_ATTN does the same with k_attn_combine's launch (gemm_fuses_attn).
 // Few rows leave each launch bound by its own start, drain and first loads:
 // three of a block's ten go, or four. One chat: hidden 576, 30 blocks and
-// head 1233 -> 1088 us, with attention's merge 1054 -> 977; hidden 5120, 4
-// blocks 501 -> 474 us.
+// head 1254 -> 1083 us, and with attention's merge, after four waves an
+// attention item, 1045 -> 977; hidden 5120, 4 blocks 502 -> 470 us.
 __device__ static inline float row_scale(const RowScale& rs, int m);
 constexpr int LX_PRO_NONE = 0, LX_PRO_RESID = 1, LX_PRO_SWIGLU = 2, LX_PRO_ATTN = 3;
 struct LxPro {
@@ -1458,8 +1458,8 @@ __device__ static inline void swiglu8(const LxPro& p, int M, int m, int k0, floa
 // Whether w's matmul at M rows forms its operand itself: yes while what each
 // workgroup then reads, its columns of `values` f32 planes of M rows, is at
 // most this. Reading it is the cost: a launch saved is about 3 us, and a
-// workgroup's share comes in at about 100 KB/us once its 511 neighbours read
-// theirs from the L2s too. Passes measured with the line swept from 0 to 4 MB,
+// workgroup's share comes in at about 100 KB/us once the launch's others (one
+// a CU at most) read theirs from the L2s too. Passes measured with the line swept from 0 to 4 MB,
 // none fused against the best line against every one fused, us:
 //   hidden 576,  8 blocks:  1 row 384/313/313, 4: 388/325/326, 16: 414/375/375
 //   hidden 4096, 4 blocks:  1 row 368/334/334, 4: 384/364/365, 8: 401/395/401,
